@@ -21,6 +21,7 @@
 #include "b2g_kernels.h"
 #include "b2g_grid.h"
 #include "b2g_partition.h"
+#include "b2g_flow.h"
 
 using namespace b2g;
 
@@ -205,6 +206,8 @@ struct b2g_batch {
   int solver_mode = 0;       // B2G_SOLVER_AUTO / _COLOURS / _WORLDS
   bool keep_idle = true;     // B2G_OPT_KEEP_IDLE
   int pair_search = 0;       // B2G_OPT_PAIR_SEARCH
+  int sweeps = 0;            // B2G_OPT_SWEEPS
+  int last_sweeps = 0;       // 1 a launch per colour, 2 ordered by data (k_flow_velocity, k_flow_position)
   int last_pair_search = 0;  // 1 LBVH, 2 grid
   int world_static_max = 0;  // most static shapes in one world
   bool grid_local_ok = false;  // every world fits a bucket table of its own (k_grid_bin_worlds)
@@ -244,6 +247,7 @@ struct b2g_batch {
   void enqueue_colour_groups();
   void enqueue_islands_and_init();
   void enqueue_islands_join();
+  void use_flow();
   void enqueue_solve(int vi, int pi, const std::vector<int>& colours, const std::vector<int>& sizes,
                      const std::vector<int>& begins, int graph_grid, bool finish_in_broadphase);
   bool finish_pending = false;  // the step's body finish is left to the broadphase's AABB launch
@@ -305,6 +309,8 @@ int b2g_batch::alloc() {
   A(d.shdr, NS); A(d.geo, 9 * (size_t)NS); A(d.smat, NS); A(d.sfilt, NS); A(d.aabb, NS);
   A(d.joints, NJ); A(d.jsol, NJ); A(d.jorder, NJ); A(d.jisland, NJ); A(d.wj_off, NW + 1); A(d.wj_list, NJ);
   A(d.bj_off, NB + 1); A(d.bj_other, 2 * NJ);
+  A(d.flow_ctl, kFlowCtl);
+  A(d.jcol_off, kMaxColours + 1); A(d.jrank, NJ); A(d.bjdeg, NB);
   A(d.ckey, NC); A(d.cpair, NC); A(d.cman, 4 * (size_t)NC); A(d.cmat, NC); A(d.ccol, NC);
   A(d.nkey, NC); A(d.npair, NC); A(d.nman, 4 * (size_t)NC); A(d.nmat, NC); A(d.ncol, NC);
   A(d.touch, NC); A(d.tpos, NC); A(d.clist, NC); A(d.cbody, NC); A(d.ccolour, NC); A(d.csorted, NC);
@@ -421,6 +427,8 @@ void b2g_batch::release() {
                   d.sort_hist, d.node_child, d.node_parent, d.leaf_parent, d.node_range, d.node_rec,
                   d.gltab, d.gloff, d.sfast, d.sparse, d.pslots, d.heavy, d.pcount, d.pfound, d.sinv, d.poff, d.poff_prev, d.scan_tiles,
                   d.cnt,
+                  // the flow solver
+                  d.fvel, d.fpos, d.flow_ctl, d.jcol_off, d.jrank, d.bjdeg,
                   // sleep
                   d.bsflag, d.bstime, d.bwake, d.bactive, d.bncontact, d.bjointed, d.isl_awake, d.isl_min, d.isl_cons,
                   // the cells solver
@@ -792,6 +800,22 @@ int b2g_batch::rebuild_joint_tables() {
   for (int c = 0; c < ncol; ++c) h_jcol_off[c + 1] += h_jcol_off[c];
   std::vector<int> cur(h_jcol_off.begin(), h_jcol_off.end());
   for (int q = 0; q < nj; ++q) order[cur[col[q]]++] = q;
+  {  // each joint's place in its bodies' update sequences (joints of a body differ in colour)
+    std::vector<int> deg(std::max(nb, 1), 0), offs(kMaxColours + 1, 0);
+    std::vector<int2> rank(std::max(nj, 1));
+    for (int k = 0; k < nj; ++k) {
+      const b2g_revolute& j = h_joints[order[k]];
+      rank[k].x = deg[j.body_a] | col[order[k]] << 8;
+      rank[k].y = deg[j.body_b];
+      ++deg[j.body_a];
+      if (j.body_b != j.body_a) ++deg[j.body_b];
+    }
+    for (int c = 0; c <= ncol; ++c) offs[c] = h_jcol_off[c];
+    d.njcol = ncol;
+    if (nb) HIP_TRY(hipMemcpy(d.bjdeg, deg.data(), nb * sizeof(int), hipMemcpyHostToDevice));
+    if (nj) HIP_TRY(hipMemcpy(d.jrank, rank.data(), nj * sizeof(int2), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(d.jcol_off, offs.data(), offs.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
   // CSR of non-colliding joint partners
   std::vector<int> off(nb + 1, 0), other;
   for (int q = 0; q < nj; ++q) {
@@ -1030,6 +1054,23 @@ void b2g_batch::enqueue_colour_groups() {
   hipLaunchKernelGGL(k_sort_serial_group, dim3(1), dim3(1), 0, stream, d);
 }
 
+// The coming step's sweeps may be ordered by data: the bodies' flow states
+// exist from the first such step on (a batch that only ever takes the
+// per-world solver does without their 256 bytes per body). Without room for
+// them the step launches its colours one by one.
+void b2g_batch::use_flow() {
+  d.flow_on = 0;
+  if (sweeps == 1) return;
+  const size_t bytes = (size_t)kFlowStride * std::max(cap.bodies, 1);
+  for (unsigned long long** p : {&d.fvel, &d.fpos})
+    if (!*p && hipMalloc((void**)p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      *p = nullptr;
+      return;
+    }
+  d.flow_on = 1;
+}
+
 // per-world island pass: LDS forest sizes (bodies); larger worlds use the
 // device-wide union-find
 constexpr int kIslandLdsSmall = 2048, kIslandLdsMid = 8192, kIslandLdsLarge = 32768;
@@ -1128,6 +1169,18 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
       ts.off[ts.n] = begins[nnorm - 1] + sizes[nnorm - 1];
     }
   }
+  // ordered by data instead (b2g_flow.h): an eager step without a serial
+  // group, of no more constraints than the launch keeps resident
+  const int flow_cons = nnorm ? begins.empty() ? 0 : begins[nnorm - 1] + sizes[nnorm - 1] : 0;
+  // constraints to a wave: few where the waves are few (kFlowSpread waves, one
+  // or two per SIMD), up to one per lane
+  const int per = std::min(kWave, std::max(1, (flow_cons + d.nj + kFlowSpread - 1) / kFlowSpread));
+  const int jblocks = (d.nj + per * kFlowWaves - 1) / (per * kFlowWaves);
+  const int flow_blocks = jblocks + (flow_cons + per * kFlowWaves - 1) / (per * kFlowWaves);
+  const bool flow = d.flow_on && !tail && !has_serial && flow_blocks <= kFlowMaxBlocks && pi <= kFlowMaxPosIters &&
+                    (nnorm == 0 || colours[nnorm - 1] < kBodyTab);
+  last_sweeps = flow ? 2 : 1;
+  const long long flow_wait = sweeps == 2 ? -1 : kFlowEnterTicks;
   auto contact_sweep = [&](int id, auto kernel, auto tail_kernel, auto... extra) {
     long long run_items = 0;
     if (tq > 0) tbegin(id);  // one timed run: the per-colour launches
@@ -1163,7 +1216,15 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
   };
   // warm start: a gather per body when every colour has a body-table entry
   const int top_colour = nnorm ? colours[nnorm - 1] : -1;
-  if (tail) {  // captured steps: the gather, then the colours past the body table and the serial group
+  if (flow) {
+    if (flow_cons > 0) {
+      const LaunchShape wg = shape_for(d.nb);
+      launch(B2G_KERNEL_WARM_START, flow_cons, k_warm_gather, wg.grid, wg.block, 0, d);
+    }
+    if (flow_blocks > 0)
+      launch(B2G_KERNEL_CONTACT_VELOCITY, (long long)flow_cons * vi, k_flow_velocity, dim3(flow_blocks),
+             dim3(kFlowThreads), 0, d, flow_cons, jblocks, per, vi, flow_wait);
+  } else if (tail) {  // captured steps: the gather, then the colours past the body table and the serial group
     const LaunchShape wg = shape_for(d.nb);
     launch(B2G_KERNEL_WARM_START, -1, k_warm_gather, wg.grid, wg.block, 0, d);
     TailSlots wt{};
@@ -1184,10 +1245,12 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
   } else {
     contact_sweep(B2G_KERNEL_WARM_START, k_warm_start, k_sweep_tail<kTailWarm>);
   }
-  joint_sweep(k_joint_init);
-  for (int it = 0; it < vi; ++it) {
-    joint_sweep(k_joint_velocity);
-    contact_sweep(B2G_KERNEL_CONTACT_VELOCITY, k_contact_velocity, k_sweep_tail<kTailVelocity>);
+  if (!flow) {
+    joint_sweep(k_joint_init);
+    for (int it = 0; it < vi; ++it) {
+      joint_sweep(k_joint_velocity);
+      contact_sweep(B2G_KERNEL_CONTACT_VELOCITY, k_contact_velocity, k_sweep_tail<kTailVelocity>);
+    }
   }
   // the island pass (side stream) ended long before the velocity phase did;
   // the same launch stores impulses, integrates positions and assigns islands
@@ -1196,7 +1259,10 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
     const LaunchShape si = shape_for(std::max(est_cons + d.nj, d.nb));
     hipLaunchKernelGGL(k_store_and_integrate, si.grid, si.block, 0, stream, d, 1);
   }
-  for (int it = 0; it < pi; ++it) {  // each launch applies the island early exit itself
+  if (flow && flow_blocks > 0 && pi > 0)
+    launch(B2G_KERNEL_CONTACT_POSITION, (long long)flow_cons * pi, k_flow_position, dim3(flow_blocks),
+           dim3(kFlowThreads), 0, d, flow_cons, jblocks, per, pi, flow_wait);
+  for (int it = 0; it < pi && !flow; ++it) {  // each launch applies the island early exit itself
     contact_sweep(B2G_KERNEL_CONTACT_POSITION, k_contact_position, k_sweep_tail<kTailPosition>, it);
     joint_sweep(k_joint_position, it);
   }
@@ -1213,6 +1279,7 @@ int b2g_batch::status_error() const {
     return fail(B2G_ERR_CAPACITY, "contact capacity exceeded (" + std::to_string(pinned[C_PAIRS]) + " pairs)");
   if (s & S_STACK_OVERFLOW) return fail(B2G_ERR_CAPACITY, "BVH traversal stack overflow");
   if (s & S_TREE_CORRUPT) return fail(B2G_ERR_INVALID, "BVH inconsistent (sort/build)");
+  if (s & S_FLOW_STALL) return fail(B2G_ERR_INVALID, "a constraint waited two seconds for its bodies");
   return B2G_OK;
 }
 
@@ -1412,6 +1479,7 @@ int b2g_batch::step(int vi, int pi, unsigned flags) {
   d.events_on = (flags & B2G_STEP_EVENTS) ? 1 : 0;
   d.sleep_on = sleep_now() ? 1 : 0;
   d.segs = 0;  // an eager step sets it once its contact list is known
+  d.flow_on = 0;  // a step by colour sweeps sets it
   const bool collide_only = (flags & B2G_STEP_COLLIDE_ONLY) != 0;
   if ((flags & B2G_STEP_SKIP_BROADPHASE) && !collide_only) {  // bodies move without a rebuild or a pair query
     tree_stale = true;
@@ -1465,6 +1533,7 @@ int b2g_batch::sleep_step(int vi, int pi, unsigned flags) {
     if ((rc = broadphase(false))) return rc;
   }
   d.segs = pairs_current && worlds_contiguous ? 1 : 0;
+  use_flow();
   hipLaunchKernelGGL(k_sleep_reset, dim3(grid_for(d.nb)), dim3(kBlock), 0, stream, d);
   enqueue_collide_and_colour_eager();
   if (prof_on) HIP_TRY(hipEventRecord(ev[1], stream));
@@ -1532,6 +1601,7 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
   // the contact list is the last broadphase's pair list: world contact
   // ranges are segment offsets
   d.segs = pairs_current && worlds_contiguous ? 1 : 0;
+  if (!use_per_world()) use_flow();
   enqueue_collide_and_colour_eager();
   if (prof_on) HIP_TRY(hipEventRecord(ev[1], stream));
   int rc;
@@ -2188,6 +2258,10 @@ int b2g_set_option(b2g_batch* b, int32_t option, int32_t value) {
       }
       b->pair_search = value;
       break;
+    case B2G_OPT_SWEEPS:
+      if (value < 0 || value > 2) return fail(B2G_ERR_INVALID, "sweeps: 0 (automatic), 1 (a launch per colour) or 2");
+      b->sweeps = value;
+      break;
     default:
       return fail(B2G_ERR_INVALID, "unknown option");
   }
@@ -2212,6 +2286,8 @@ int b2g_get_option(b2g_batch* b, int32_t option, int32_t* value) {
     case B2G_OPT_KEEP_IDLE: *value = b->keep_idle ? 1 : 0; break;
     case B2G_OPT_PAIR_SEARCH: *value = b->pair_search; break;
     case B2G_OPT_LAST_PAIR_SEARCH: *value = b->last_pair_search; break;
+    case B2G_OPT_SWEEPS: *value = b->sweeps; break;
+    case B2G_OPT_LAST_SWEEPS: *value = b->last_sweeps; break;
     default: return fail(B2G_ERR_INVALID, "unknown option");
   }
   return B2G_OK;

@@ -52,7 +52,7 @@ enum Counter : int {
   C_PART_CROSS = 13,  // constraints of the cells solver's cross group this step
   C_COUNT = 16
 };
-enum Status : int { S_CONTACT_OVERFLOW = 1, S_STACK_OVERFLOW = 2, S_TREE_CORRUPT = 4, S_EVENT_OVERFLOW = 8 };
+enum Status : int { S_CONTACT_OVERFLOW = 1, S_STACK_OVERFLOW = 2, S_TREE_CORRUPT = 4, S_EVENT_OVERFLOW = 8, S_FLOW_STALL = 16 };
 // contact event kinds: touching began / ended in Collide, touching contact
 // destroyed by the broadphase (b2ContactManager::Destroy)
 enum EventKind : int { kEventBegin = 1, kEventEnd = 2, kEventDestroyed = 3 };
@@ -65,6 +65,11 @@ constexpr int kBodyTab = 32;
 constexpr int kCntColOff = 32;  // the colour offsets sit this many ints into the counter block  // colours a body's warm-start gather covers
 
 // all device arrays, passed by value to every kernel
+constexpr int kFlowCtl = 64;
+// bytes from one body's flow state to the next: a cache line each (16 bytes,
+// eight bodies to a line: 322 us per velocity phase of a settled pile of
+// 20,000 against 242)
+constexpr int kFlowStride = 128;
 struct Dev {
   int nb, ns, nj, nw;
   // bodies
@@ -210,6 +215,16 @@ struct Dev {
   int* part_coff;     // kPartGroups * (kColourSlots + 1): slot offsets of each group's colours
   unsigned long long* part_claim;  // per body: colouring claims of the cross group
   unsigned long long* part_used;   // per body: colours the cross group gave its constraints
+  // the flow solver (b2g_flow.h)
+  int flow_on;        // this step may solve by k_flow_velocity / k_flow_position
+  unsigned long long* fvel;  // 2 per body: velocity, each word with a 16-bit update count
+  unsigned long long* fpos;  // 2 per body: centre and angle, the same way
+  int* flow_ctl;      // kFlowCtl words: arrival counts and go words of the step's flow launches
+  int* jcol_off;      // offsets of the joint colours (kMaxColours + 1)
+  int njcol;          // joint colours
+  int2* jrank;        // per colour-ordered joint: its place among each body's joints, in colour order (x: its
+                      // colour above bit 8)
+  int* bjdeg;         // per body: joints attached to it
   int* part_xcol;     // per cross-group constraint: its colour while colouring
   int2* sloc;         // per slot: LDS slots of its two bodies in its cell (-1: global memory)
 };
@@ -310,6 +325,7 @@ __global__ void k_events_reset(Dev d) {
 // the step's colour counters (block 0 of the launch that integrates velocities)
 __device__ __forceinline__ void reset_colour_counters(const Dev& d) {
   for (int c = threadIdx.x; c < kColourSlots; c += blockDim.x) d.col_count[c] = 0;
+  if (threadIdx.x < kFlowCtl) d.flow_ctl[threadIdx.x] = 0;
   if (threadIdx.x == 0) {
     d.cnt[C_REMAIN] = 0;
     d.cnt[C_PENDING] = 0;
@@ -325,6 +341,22 @@ __device__ __forceinline__ bool body_awake0(const Dev& d, int b) {
   return d.btype[b] != kStaticBody && (d.bsflag[b] & kBodyAsleep) == 0;
 }
 __device__ __forceinline__ bool world_sleeps(const Dev& d, int w) { return (d.wflag[w] & 4) != 0; }
+
+// A body's three state floats for the flow solver: two 64-bit words, each
+// with 16 bits of the body's update count on top (the third float is split
+// over the two), so a reader that finds the count it waits for in both words
+// holds one consistent state, whatever order the words arrive in.
+__device__ __forceinline__ void flow_pack(float x, float y, float z, unsigned count, unsigned long long* w) {
+  const unsigned zb = as_uint(z);
+  w[0] = (unsigned long long)as_uint(x) | ((unsigned long long)((zb >> 16) | (count << 16)) << 32);
+  w[1] = (unsigned long long)as_uint(y) | ((unsigned long long)((zb & 0xffffu) | (count << 16)) << 32);
+}
+// a body's state before its first update of the phase
+__device__ __forceinline__ void flow_start(unsigned long long* state, int b, float x, float y, float z) {
+  unsigned long long w[2];
+  flow_pack(x, y, z, 0u, w);
+  *reinterpret_cast<ulonglong2*>(state + (kFlowStride / 8) * (size_t)b) = make_ulonglong2(w[0], w[1]);
+}
 
 // integrate = 1: the step's per-body resets and the velocity integration;
 // 0: the resets only (the integration follows the islands, which decide which
@@ -355,6 +387,7 @@ __device__ __forceinline__ void integrate_velocity(const Dev& d, int b, int inte
     vy = vy / ld;
     w_ = w_ / ad;
     d.vel[b] = make_float4(vx, vy, w_, 0.0f);
+    if (d.flow_on) flow_start(d.fvel, b, vx, vy, w_);
   }
 }
 
@@ -1009,6 +1042,10 @@ __device__ __forceinline__ void island_reset(const Dev& d, int isl) {
   d.solved[isl] = 0;
   d.sepbad[isl] = 0u;
   d.jok[isl] = 1;
+  if (d.flow_on) {  // (the flow solver clears no slot ahead during the first three iterations)
+    d.sepbad[(size_t)d.nb + isl] = d.sepbad[2 * (size_t)d.nb + isl] = 0u;
+    d.jok[(size_t)d.nb + isl] = d.jok[2 * (size_t)d.nb + isl] = 1;
+  }
 }
 
 // Per-island early exit (b2_island.cpp:403-408): an island stops after the
@@ -1245,31 +1282,40 @@ struct LdsBodies {
   __device__ __forceinline__ bool writes(const Dev& d, int i) const { return writes_body(d, i); }
 };
 
+// Both bodies' velocities around one constraint's update.
+struct VelPair {
+  vec2 vA, vB;
+  float wA, wB;
+};
+__device__ __forceinline__ VelPair vel_pair(float4 a, float4 b) {
+  return VelPair{mk(a.x, a.y), mk(b.x, b.y), a.z, b.z};
+}
+// (`src` gives the constraint's fields)
+template <class Src>
+__device__ __forceinline__ void warm_start_core(const Src& src, int count, VelPair& u) {
+  const float4 n4 = src.vc(0), m = src.vc(1);
+  const vec2 normal = mk(n4.x, n4.y), tangent = cross(normal, 1.0f);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (j < count) {
+      const float4 r = src.vc(3 + 2 * j), im = src.vc(4 + 2 * j);
+      const vec2 P = im.x * normal + im.y * tangent;
+      u.wA -= m.z * cross(mk(r.x, r.y), P);
+      u.vA = u.vA - m.x * P;
+      u.wB += m.w * cross(mk(r.z, r.w), P);
+      u.vB = u.vB + m.y * P;
+    }
+  }
+}
 template <class BV, class Src>
 __device__ __forceinline__ void warm_start_src(const Dev& d, BV vel, const Src& src) {
-  {
-    const float4 v2i = src.vc(2);
-    const int ia = as_int(v2i.x), ib = as_int(v2i.y), count = as_int(v2i.z) & 0xff;
-    if ((as_int(v2i.z) & 256) == 0) return;  // no warm starting in this world
-    const float4 n4 = src.vc(0), m = src.vc(1);
-    const vec2 normal = mk(n4.x, n4.y), tangent = cross(normal, 1.0f);
-    float4 va = *vel(ia), vb = *vel(ib);
-    vec2 vA = mk(va.x, va.y), vB = mk(vb.x, vb.y);
-    float wA = va.z, wB = vb.z;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (j < count) {
-        const float4 r = src.vc(3 + 2 * j), im = src.vc(4 + 2 * j);
-        const vec2 P = im.x * normal + im.y * tangent;
-        wA -= m.z * cross(mk(r.x, r.y), P);
-        vA = vA - m.x * P;
-        wB += m.w * cross(mk(r.z, r.w), P);
-        vB = vB + m.y * P;
-      }
-    }
-    if (vel.writes(d, ia)) *vel(ia) = make_float4(vA.x, vA.y, wA, 0.0f);
-    if (vel.writes(d, ib)) *vel(ib) = make_float4(vB.x, vB.y, wB, 0.0f);
-  }
+  const float4 v2i = src.vc(2);
+  const int ia = as_int(v2i.x), ib = as_int(v2i.y), count = as_int(v2i.z) & 0xff;
+  if ((as_int(v2i.z) & 256) == 0) return;  // no warm starting in this world
+  VelPair u = vel_pair(*vel(ia), *vel(ib));
+  warm_start_core(src, count, u);
+  if (vel.writes(d, ia)) *vel(ia) = make_float4(u.vA.x, u.vA.y, u.wA, 0.0f);
+  if (vel.writes(d, ib)) *vel(ib) = make_float4(u.vB.x, u.vB.y, u.wB, 0.0f);
 }
 
 // b2ContactSolver::SolveVelocityConstraints (:301-639) for slots [begin, end)
@@ -1338,23 +1384,20 @@ __device__ __forceinline__ PositionRegs load_position_regs(const Dev& d, int s) 
   return r;
 }
 
-template <class BV, class Src>
-__device__ __forceinline__ void contact_velocity_src(const Dev& d, int s, BV vel, const Src& src) {
-  const float4 v2i = src.vc(2);
-  const int ia = as_int(v2i.x), ib = as_int(v2i.y), count = as_int(v2i.z) & 0xff;
-  if (count == 0) return;  // a constraint of a sleeping island
+// One velocity update of a contact of `count` (1 or 2) points: bodies `u`, the
+// points' impulses and masses q0, q1 (fields 4 and 6), the rest from `src`.
+template <class Src>
+__device__ __forceinline__ void contact_velocity_core(const Src& src, int count, VelPair& u, float4& q0, float4& q1) {
   const float4 n4 = src.vc(0), m = src.vc(1);
   const float mA = m.x, mB = m.y, iA = m.z, iB = m.w;
   const vec2 normal = mk(n4.x, n4.y);
   const float friction = n4.z, tangent_speed = n4.w;
-  float4 va = *vel(ia), vb = *vel(ib);
-  vec2 vA = mk(va.x, va.y), vB = mk(vb.x, vb.y);
-  float wA = va.z, wB = vb.z;
   const float4 r0 = src.vc(3), r1 = src.vc(5);
-  float4 q0 = src.vc(4), q1 = src.vc(6);
   const vec2 rA0 = mk(r0.x, r0.y), rB0 = mk(r0.z, r0.w);
   const vec2 rA1 = mk(r1.x, r1.y), rB1 = mk(r1.z, r1.w);
   const vec2 tangent = cross(normal, 1.0f);
+  vec2 vA = u.vA, vB = u.vB;
+  float wA = u.wA, wB = u.wB;
   // friction first (:324-351)
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -1435,9 +1478,22 @@ __device__ __forceinline__ void contact_velocity_src(const Dev& d, int s, BV vel
       q1.x = x.y;
     }
   }
+  u.vA = vA;
+  u.vB = vB;
+  u.wA = wA;
+  u.wB = wB;
+}
+template <class BV, class Src>
+__device__ __forceinline__ void contact_velocity_src(const Dev& d, int s, BV vel, const Src& src) {
+  const float4 v2i = src.vc(2);
+  const int ia = as_int(v2i.x), ib = as_int(v2i.y), count = as_int(v2i.z) & 0xff;
+  if (count == 0) return;  // a constraint of a sleeping island
+  VelPair u = vel_pair(*vel(ia), *vel(ib));
+  float4 q0 = src.vc(4), q1 = src.vc(6);
+  contact_velocity_core(src, count, u, q0, q1);
   src.put_impulses(d, s, q0, q1, count);
-  if (vel.writes(d, ia)) *vel(ia) = make_float4(vA.x, vA.y, wA, 0.0f);
-  if (vel.writes(d, ib)) *vel(ib) = make_float4(vB.x, vB.y, wB, 0.0f);
+  if (vel.writes(d, ia)) *vel(ia) = make_float4(u.vA.x, u.vA.y, u.wA, 0.0f);
+  if (vel.writes(d, ib)) *vel(ib) = make_float4(u.vB.x, u.vB.y, u.wB, 0.0f);
 }
 template <class BV>
 __device__ __forceinline__ void contact_velocity_t(const Dev& d, int s, BV vel) {
@@ -1521,6 +1577,7 @@ __device__ __forceinline__ void integrate_position(const Dev& d, int b) {
     const float a = p.z + h * wv;
     d.pos[b] = make_float4(c.x, c.y, a, 0.0f);
     d.vel[b] = make_float4(v.x, v.y, wv, 0.0f);
+    if (d.flow_on) flow_start(d.fpos, b, c.x, c.y, a);
   }
 }
 
@@ -1541,23 +1598,24 @@ __global__ void __launch_bounds__(kBlock) k_store_and_integrate(Dev d, int islan
 
 // b2ContactSolver::SolvePositionConstraints (:659-787) for slots [begin, end)
 // returns the minimum separation seen (0 when the island is already solved)
-template <class BP, class Src>
-__device__ __forceinline__ float contact_position_src(const Dev& d, int isl, int it, BP pos, const Src& src) {
-  // the constraint's loads are issued before the island test, so they are in
-  // flight together with it
-  const float4 v2i = src.vc(2);
-  const float4 q0 = src.pc(0), q1 = src.pc(1), q2 = src.pc(2), q3 = src.pc(3), q4 = src.pc(4);
-  const int ia = as_int(v2i.x), ib = as_int(v2i.y);
-  const float4 pa = *pos(ia), pb = *pos(ib);  // in flight with the island test too
-  if (as_int(q4.w) == 0) return 0.0f;  // a constraint of a sleeping island
-  if (src.island_skip(d, isl, it)) return 0.0f;
+struct PosPair {
+  vec2 cA, cB;
+  float aA, aB;
+};
+__device__ __forceinline__ PosPair pos_pair(float4 a, float4 b) {
+  return PosPair{mk(a.x, a.y), mk(b.x, b.y), a.z, b.z};
+}
+// One position update of a contact (q0 .. q4: its fields pc 0 .. 4); returns
+// the least separation of its points.
+__device__ __forceinline__ float contact_position_core(float4 q0, float4 q1, float4 q2, float4 q3, float4 q4,
+                                                       PosPair& u) {
   const vec2 lp = mk(q0.x, q0.y), ln = mk(q0.z, q0.w);
   const vec2 lcA = mk(q2.x, q2.y), lcB = mk(q2.z, q2.w);
   const float mA = q3.x, mB = q3.y, iA = q3.z, iB = q3.w;
   const float radA = q4.x, radB = q4.y;
   const int mtype = as_int(q4.z), count = as_int(q4.w);
-  vec2 cA = mk(pa.x, pa.y), cB = mk(pb.x, pb.y);
-  float aA = pa.z, aB = pb.z;
+  vec2 cA = u.cA, cB = u.cB;
+  float aA = u.aA, aB = u.aB;
   float min_sep = 0.0f;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -1603,8 +1661,26 @@ __device__ __forceinline__ float contact_position_src(const Dev& d, int isl, int
       aB += iB * cross(rB, P);
     }
   }
-  if (pos.writes(d, ia)) *pos(ia) = make_float4(cA.x, cA.y, aA, 0.0f);
-  if (pos.writes(d, ib)) *pos(ib) = make_float4(cB.x, cB.y, aB, 0.0f);
+  u.cA = cA;
+  u.cB = cB;
+  u.aA = aA;
+  u.aB = aB;
+  return min_sep;
+}
+template <class BP, class Src>
+__device__ __forceinline__ float contact_position_src(const Dev& d, int isl, int it, BP pos, const Src& src) {
+  // the constraint's loads are issued before the island test, so they are in
+  // flight together with it
+  const float4 v2i = src.vc(2);
+  const float4 q0 = src.pc(0), q1 = src.pc(1), q2 = src.pc(2), q3 = src.pc(3), q4 = src.pc(4);
+  const int ia = as_int(v2i.x), ib = as_int(v2i.y);
+  const float4 pa = *pos(ia), pb = *pos(ib);  // in flight with the island test too
+  if (as_int(q4.w) == 0) return 0.0f;  // a constraint of a sleeping island
+  if (src.island_skip(d, isl, it)) return 0.0f;
+  PosPair u = pos_pair(pa, pb);
+  const float min_sep = contact_position_core(q0, q1, q2, q3, q4, u);
+  if (pos.writes(d, ia)) *pos(ia) = make_float4(u.cA.x, u.cA.y, u.aA, 0.0f);
+  if (pos.writes(d, ib)) *pos(ib) = make_float4(u.cB.x, u.cB.y, u.aB, 0.0f);
   return min_sep;
 }
 template <class BP>
@@ -1718,7 +1794,10 @@ __global__ void __launch_bounds__(kBlock) k_warm_gather(Dev d) {
         }
       }
     }
-    if (touched) d.vel[b] = make_float4(v.x, v.y, w, 0.0f);
+    if (touched) {
+      d.vel[b] = make_float4(v.x, v.y, w, 0.0f);
+      if (d.flow_on) flow_start(d.fvel, b, v.x, v.y, w);
+    }
   }
 }
 
@@ -1856,180 +1935,205 @@ __global__ void __launch_bounds__(kBlock) k_joint_prepare(Dev d) {
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_joint_init(Dev d, int begin, int end) {
-  B2G_FOR(q, begin, end) {
-    if (d.jisland[q] < 0) continue;
-    const int ji = d.jorder[q];
-    Joint j = d.joints[ji];
-    JointSolve s;
-    const float4 pa = d.prop[j.a], pb = d.prop[j.b];
-    s.lca_x = pa.z; s.lca_y = pa.w; s.lcb_x = pb.z; s.lcb_y = pb.w;
-    s.ma = pa.x; s.mb = pb.x; s.ia = pa.y; s.ib = pb.y;
-    const float aA = d.pos[j.a].z, aB = d.pos[j.b].z;
-    const float4 va = d.vel[j.a], vb = d.vel[j.b];
-    vec2 vA = mk(va.x, va.y), vB = mk(vb.x, vb.y);
-    float wA = va.z, wB = vb.z;
-    const rot2 qA = rot_of(aA), qB = rot_of(aB);
-    const vec2 rA = mul(qA, mk(j.la_x, j.la_y) - mk(s.lca_x, s.lca_y));
-    const vec2 rB = mul(qB, mk(j.lb_x, j.lb_y) - mk(s.lcb_x, s.lcb_y));
-    s.ra_x = rA.x; s.ra_y = rA.y; s.rb_x = rB.x; s.rb_y = rB.y;
-    const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
-    s.kxx = mA + mB + rA.y * rA.y * iA + rB.y * rB.y * iB;
-    s.kyx = -rA.y * rA.x * iA - rB.y * rB.x * iB;
-    s.kxy = s.kyx;
-    s.kyy = mA + mB + rA.x * rA.x * iA + rB.x * rB.x * iB;
-    s.axial = iA + iB;
-    bool fixed_rotation;
-    if (s.axial > 0.0f) {
-      s.axial = 1.0f / s.axial;
-      fixed_rotation = false;
-    } else {
-      fixed_rotation = true;
-    }
-    s.angle = aB - aA - j.ref;
-    if ((j.flags & 2) == 0 || fixed_rotation) {
-      j.lower_imp = 0.0f;
-      j.upper_imp = 0.0f;
-    }
-    if ((j.flags & 4) == 0 || fixed_rotation) j.motor = 0.0f;
-    const float4 wp = d.wpar[j.world];
-    if (d.wflag[j.world] & 1) {
-      const float r = wp.w;
-      j.imp_x *= r;
-      j.imp_y *= r;
-      j.motor *= r;
-      j.lower_imp *= r;
-      j.upper_imp *= r;
-      const float axial_impulse = j.motor + j.lower_imp - j.upper_imp;
-      const vec2 P = mk(j.imp_x, j.imp_y);
-      vA = vA - mA * P;
-      wA -= iA * (cross(rA, P) + axial_impulse);
-      vB = vB + mB * P;
-      wB += iB * (cross(rB, P) + axial_impulse);
-    } else {
-      j.imp_x = j.imp_y = 0.0f;
-      j.motor = j.lower_imp = j.upper_imp = 0.0f;
-    }
-    d.joints[ji] = j;
-    d.jsol[q] = s;
-    if (writes_body(d, j.a)) d.vel[j.a] = make_float4(vA.x, vA.y, wA, 0.0f);
-    if (writes_body(d, j.b)) d.vel[j.b] = make_float4(vB.x, vB.y, wB, 0.0f);
+// A joint's set-up and warm start (InitVelocityConstraints) on bodies at
+// angles aA, aB with mass data pa, pb.
+__device__ __forceinline__ void joint_init_core(Joint& j, JointSolve& s, float4 pa, float4 pb, float aA, float aB,
+                                                bool warm, float ratio, VelPair& u) {
+  vec2 vA = u.vA, vB = u.vB;
+  float wA = u.wA, wB = u.wB;
+  s.lca_x = pa.z; s.lca_y = pa.w; s.lcb_x = pb.z; s.lcb_y = pb.w;
+  s.ma = pa.x; s.mb = pb.x; s.ia = pa.y; s.ib = pb.y;
+  const rot2 qA = rot_of(aA), qB = rot_of(aB);
+  const vec2 rA = mul(qA, mk(j.la_x, j.la_y) - mk(s.lca_x, s.lca_y));
+  const vec2 rB = mul(qB, mk(j.lb_x, j.lb_y) - mk(s.lcb_x, s.lcb_y));
+  s.ra_x = rA.x; s.ra_y = rA.y; s.rb_x = rB.x; s.rb_y = rB.y;
+  const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
+  s.kxx = mA + mB + rA.y * rA.y * iA + rB.y * rB.y * iB;
+  s.kyx = -rA.y * rA.x * iA - rB.y * rB.x * iB;
+  s.kxy = s.kyx;
+  s.kyy = mA + mB + rA.x * rA.x * iA + rB.x * rB.x * iB;
+  s.axial = iA + iB;
+  bool fixed_rotation;
+  if (s.axial > 0.0f) {
+    s.axial = 1.0f / s.axial;
+    fixed_rotation = false;
+  } else {
+    fixed_rotation = true;
   }
+  s.angle = aB - aA - j.ref;
+  if ((j.flags & 2) == 0 || fixed_rotation) {
+    j.lower_imp = 0.0f;
+    j.upper_imp = 0.0f;
+  }
+  if ((j.flags & 4) == 0 || fixed_rotation) j.motor = 0.0f;
+  if (warm) {
+    const float r = ratio;
+    j.imp_x *= r;
+    j.imp_y *= r;
+    j.motor *= r;
+    j.lower_imp *= r;
+    j.upper_imp *= r;
+    const float axial_impulse = j.motor + j.lower_imp - j.upper_imp;
+    const vec2 P = mk(j.imp_x, j.imp_y);
+    vA = vA - mA * P;
+    wA -= iA * (cross(rA, P) + axial_impulse);
+    vB = vB + mB * P;
+    wB += iB * (cross(rB, P) + axial_impulse);
+  } else {
+    j.imp_x = j.imp_y = 0.0f;
+    j.motor = j.lower_imp = j.upper_imp = 0.0f;
+  }
+  u.vA = vA;
+  u.vB = vB;
+  u.wA = wA;
+  u.wB = wB;
 }
-
-__global__ void __launch_bounds__(kBlock) k_joint_velocity(Dev d, int begin, int end) {
-  B2G_FOR(q, begin, end) {
-    if (d.jisland[q] < 0) continue;
-    const int ji = d.jorder[q];
-    Joint j = d.joints[ji];
-    const JointSolve s = d.jsol[q];
-    const float4 va = d.vel[j.a], vb = d.vel[j.b];
-    vec2 vA = mk(va.x, va.y), vB = mk(vb.x, vb.y);
-    float wA = va.z, wB = vb.z;
-    const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
-    const bool fixed_rotation = (iA + iB == 0.0f);
-    const float4 wp = d.wpar[j.world];
-    const float h = wp.z;
-    const float inv_dt = h > 0.0f ? 1.0f / h : 0.0f;
-    if ((j.flags & 4) && !fixed_rotation) {
-      const float Cdot = wB - wA - j.speed;
-      float impulse = -s.axial * Cdot;
-      const float old = j.motor;
-      const float max_impulse = h * j.max_torque;
-      j.motor = clampf(j.motor + impulse, -max_impulse, max_impulse);
-      impulse = j.motor - old;
+// One velocity update of a joint (SolveVelocityConstraints); h: the time step.
+__device__ __forceinline__ void joint_velocity_core(Joint& j, const JointSolve& s, float h, VelPair& u) {
+  vec2 vA = u.vA, vB = u.vB;
+  float wA = u.wA, wB = u.wB;
+  const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
+  const bool fixed_rotation = (iA + iB == 0.0f);
+  const float inv_dt = h > 0.0f ? 1.0f / h : 0.0f;
+  if ((j.flags & 4) && !fixed_rotation) {
+    const float Cdot = wB - wA - j.speed;
+    float impulse = -s.axial * Cdot;
+    const float old = j.motor;
+    const float max_impulse = h * j.max_torque;
+    j.motor = clampf(j.motor + impulse, -max_impulse, max_impulse);
+    impulse = j.motor - old;
+    wA -= iA * impulse;
+    wB += iB * impulse;
+  }
+  if ((j.flags & 2) && !fixed_rotation) {
+    {
+      const float C = s.angle - j.lower;
+      const float Cdot = wB - wA;
+      float impulse = -s.axial * (Cdot + maxf(C, 0.0f) * inv_dt);
+      const float old = j.lower_imp;
+      j.lower_imp = maxf(j.lower_imp + impulse, 0.0f);
+      impulse = j.lower_imp - old;
       wA -= iA * impulse;
       wB += iB * impulse;
     }
-    if ((j.flags & 2) && !fixed_rotation) {
-      {
-        const float C = s.angle - j.lower;
-        const float Cdot = wB - wA;
-        float impulse = -s.axial * (Cdot + maxf(C, 0.0f) * inv_dt);
-        const float old = j.lower_imp;
-        j.lower_imp = maxf(j.lower_imp + impulse, 0.0f);
-        impulse = j.lower_imp - old;
-        wA -= iA * impulse;
-        wB += iB * impulse;
-      }
-      {
-        const float C = j.upper - s.angle;
-        const float Cdot = wA - wB;
-        float impulse = -s.axial * (Cdot + maxf(C, 0.0f) * inv_dt);
-        const float old = j.upper_imp;
-        j.upper_imp = maxf(j.upper_imp + impulse, 0.0f);
-        impulse = j.upper_imp - old;
-        wA += iA * impulse;
-        wB -= iB * impulse;
-      }
-    }
     {
-      const vec2 rA = mk(s.ra_x, s.ra_y), rB = mk(s.rb_x, s.rb_y);
-      const vec2 Cdot = vB + cross(wB, rB) - vA - cross(wA, rA);
-      const mat22 K = {mk(s.kxx, s.kxy), mk(s.kyx, s.kyy)};
-      const vec2 impulse = solve(K, -Cdot);
-      j.imp_x += impulse.x;
-      j.imp_y += impulse.y;
-      vA = vA - mA * impulse;
-      wA -= iA * cross(rA, impulse);
-      vB = vB + mB * impulse;
-      wB += iB * cross(rB, impulse);
+      const float C = j.upper - s.angle;
+      const float Cdot = wA - wB;
+      float impulse = -s.axial * (Cdot + maxf(C, 0.0f) * inv_dt);
+      const float old = j.upper_imp;
+      j.upper_imp = maxf(j.upper_imp + impulse, 0.0f);
+      impulse = j.upper_imp - old;
+      wA += iA * impulse;
+      wB -= iB * impulse;
     }
-    d.joints[ji] = j;
-    if (writes_body(d, j.a)) d.vel[j.a] = make_float4(vA.x, vA.y, wA, 0.0f);
-    if (writes_body(d, j.b)) d.vel[j.b] = make_float4(vB.x, vB.y, wB, 0.0f);
   }
+  {
+    const vec2 rA = mk(s.ra_x, s.ra_y), rB = mk(s.rb_x, s.rb_y);
+    const vec2 Cdot = vB + cross(wB, rB) - vA - cross(wA, rA);
+    const mat22 K = {mk(s.kxx, s.kxy), mk(s.kyx, s.kyy)};
+    const vec2 impulse = solve(K, -Cdot);
+    j.imp_x += impulse.x;
+    j.imp_y += impulse.y;
+    vA = vA - mA * impulse;
+    wA -= iA * cross(rA, impulse);
+    vB = vB + mB * impulse;
+    wB += iB * cross(rB, impulse);
+  }
+  u.vA = vA;
+  u.vB = vB;
+  u.wA = wA;
+  u.wB = wB;
+}
+// One position update of a joint (SolvePositionConstraints); true when the
+// joint was within its slop.
+__device__ __forceinline__ bool joint_position_core(const Joint& j, const JointSolve& s, PosPair& u) {
+  vec2 cA = u.cA, cB = u.cB;
+  float aA = u.aA, aB = u.aB;
+  float angular_error = 0.0f, position_error = 0.0f;
+  const bool fixed_rotation = (s.ia + s.ib == 0.0f);
+  if ((j.flags & 2) && !fixed_rotation) {
+    const float angle = aB - aA - j.ref;
+    float C = 0.0f;
+    if (absf(j.upper - j.lower) < 2.0f * kAngularSlop)
+      C = clampf(angle - j.lower, -kMaxAngularCorrection, kMaxAngularCorrection);
+    else if (angle <= j.lower)
+      C = clampf(angle - j.lower + kAngularSlop, -kMaxAngularCorrection, 0.0f);
+    else if (angle >= j.upper)
+      C = clampf(angle - j.upper - kAngularSlop, 0.0f, kMaxAngularCorrection);
+    const float limit_impulse = -s.axial * C;
+    aA -= s.ia * limit_impulse;
+    aB += s.ib * limit_impulse;
+    angular_error = absf(C);
+  }
+  {
+    const rot2 qA = rot_of(aA), qB = rot_of(aB);
+    const vec2 rA = mul(qA, mk(j.la_x, j.la_y) - mk(s.lca_x, s.lca_y));
+    const vec2 rB = mul(qB, mk(j.lb_x, j.lb_y) - mk(s.lcb_x, s.lcb_y));
+    const vec2 C = cB + rB - cA - rA;
+    position_error = length(C);
+    const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
+    mat22 K;
+    K.ex.x = mA + mB + iA * rA.y * rA.y + iB * rB.y * rB.y;
+    K.ex.y = -iA * rA.x * rA.y - iB * rB.x * rB.y;
+    K.ey.x = K.ex.y;
+    K.ey.y = mA + mB + iA * rA.x * rA.x + iB * rB.x * rB.x;
+    const vec2 impulse = -solve(K, C);
+    cA = cA - mA * impulse;
+    aA -= iA * cross(rA, impulse);
+    cB = cB + mB * impulse;
+    aB += iB * cross(rB, impulse);
+  }
+  u.cA = cA;
+  u.cB = cB;
+  u.aA = aA;
+  u.aB = aB;
+  return position_error <= kLinearSlop && angular_error <= kAngularSlop;
 }
 
+__device__ __forceinline__ void joint_init(const Dev& d, int q) {
+  if (d.jisland[q] < 0) return;
+  const int ji = d.jorder[q];
+  Joint j = d.joints[ji];
+  JointSolve s{};
+  VelPair u = vel_pair(d.vel[j.a], d.vel[j.b]);
+  joint_init_core(j, s, d.prop[j.a], d.prop[j.b], d.pos[j.a].z, d.pos[j.b].z, (d.wflag[j.world] & 1) != 0,
+                  d.wpar[j.world].w, u);
+  d.joints[ji] = j;
+  d.jsol[q] = s;
+  if (writes_body(d, j.a)) d.vel[j.a] = make_float4(u.vA.x, u.vA.y, u.wA, 0.0f);
+  if (writes_body(d, j.b)) d.vel[j.b] = make_float4(u.vB.x, u.vB.y, u.wB, 0.0f);
+}
+__device__ __forceinline__ void joint_velocity(const Dev& d, int q) {
+  if (d.jisland[q] < 0) return;
+  const int ji = d.jorder[q];
+  Joint j = d.joints[ji];
+  const JointSolve s = d.jsol[q];
+  VelPair u = vel_pair(d.vel[j.a], d.vel[j.b]);
+  joint_velocity_core(j, s, d.wpar[j.world].z, u);
+  d.joints[ji] = j;
+  if (writes_body(d, j.a)) d.vel[j.a] = make_float4(u.vA.x, u.vA.y, u.wA, 0.0f);
+  if (writes_body(d, j.b)) d.vel[j.b] = make_float4(u.vB.x, u.vB.y, u.wB, 0.0f);
+}
+__device__ __forceinline__ void joint_position(const Dev& d, int q, int it) {
+  const int isl = d.jisland[q];
+  if (isl < 0 || island_done(d, isl, it)) return;
+  island_rearm(d, isl, it);
+  const Joint j = d.joints[d.jorder[q]];
+  const JointSolve s = d.jsol[q];
+  PosPair u = pos_pair(d.pos[j.a], d.pos[j.b]);
+  const bool ok = joint_position_core(j, s, u);
+  if (writes_body(d, j.a)) d.pos[j.a] = make_float4(u.cA.x, u.cA.y, u.aA, 0.0f);
+  if (writes_body(d, j.b)) d.pos[j.b] = make_float4(u.cB.x, u.cB.y, u.aB, 0.0f);
+  if (!ok) d.jok[island_slot(d, isl, it)] = 0;
+}
+__global__ void __launch_bounds__(kBlock) k_joint_init(Dev d, int begin, int end) {
+  B2G_FOR(q, begin, end) joint_init(d, q);
+}
+__global__ void __launch_bounds__(kBlock) k_joint_velocity(Dev d, int begin, int end) {
+  B2G_FOR(q, begin, end) joint_velocity(d, q);
+}
 __global__ void __launch_bounds__(kBlock) k_joint_position(Dev d, int begin, int end, int it) {
-  B2G_FOR(q, begin, end) {
-    const int isl = d.jisland[q];
-    if (isl < 0 || island_done(d, isl, it)) continue;
-    island_rearm(d, isl, it);
-    const Joint j = d.joints[d.jorder[q]];
-    const JointSolve s = d.jsol[q];
-    const float4 pa = d.pos[j.a], pb = d.pos[j.b];
-    vec2 cA = mk(pa.x, pa.y), cB = mk(pb.x, pb.y);
-    float aA = pa.z, aB = pb.z;
-    float angular_error = 0.0f, position_error = 0.0f;
-    const bool fixed_rotation = (s.ia + s.ib == 0.0f);
-    if ((j.flags & 2) && !fixed_rotation) {
-      const float angle = aB - aA - j.ref;
-      float C = 0.0f;
-      if (absf(j.upper - j.lower) < 2.0f * kAngularSlop)
-        C = clampf(angle - j.lower, -kMaxAngularCorrection, kMaxAngularCorrection);
-      else if (angle <= j.lower)
-        C = clampf(angle - j.lower + kAngularSlop, -kMaxAngularCorrection, 0.0f);
-      else if (angle >= j.upper)
-        C = clampf(angle - j.upper - kAngularSlop, 0.0f, kMaxAngularCorrection);
-      const float limit_impulse = -s.axial * C;
-      aA -= s.ia * limit_impulse;
-      aB += s.ib * limit_impulse;
-      angular_error = absf(C);
-    }
-    {
-      const rot2 qA = rot_of(aA), qB = rot_of(aB);
-      const vec2 rA = mul(qA, mk(j.la_x, j.la_y) - mk(s.lca_x, s.lca_y));
-      const vec2 rB = mul(qB, mk(j.lb_x, j.lb_y) - mk(s.lcb_x, s.lcb_y));
-      const vec2 C = cB + rB - cA - rA;
-      position_error = length(C);
-      const float mA = s.ma, mB = s.mb, iA = s.ia, iB = s.ib;
-      mat22 K;
-      K.ex.x = mA + mB + iA * rA.y * rA.y + iB * rB.y * rB.y;
-      K.ex.y = -iA * rA.x * rA.y - iB * rB.x * rB.y;
-      K.ey.x = K.ex.y;
-      K.ey.y = mA + mB + iA * rA.x * rA.x + iB * rB.x * rB.x;
-      const vec2 impulse = -solve(K, C);
-      cA = cA - mA * impulse;
-      aA -= iA * cross(rA, impulse);
-      cB = cB + mB * impulse;
-      aB += iB * cross(rB, impulse);
-    }
-    if (writes_body(d, j.a)) d.pos[j.a] = make_float4(cA.x, cA.y, aA, 0.0f);
-    if (writes_body(d, j.b)) d.pos[j.b] = make_float4(cB.x, cB.y, aB, 0.0f);
-    const bool ok = position_error <= kLinearSlop && angular_error <= kAngularSlop;
-    if (!ok) d.jok[island_slot(d, isl, it)] = 0;
-  }
+  B2G_FOR(q, begin, end) joint_position(d, q, it);
 }
 
 // Island of every solved contact slot and joint, and the island's position

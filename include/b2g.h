@@ -319,7 +319,18 @@ enum {
    * the LBVH. The pair list is the same either way. B2G_OPT_LAST_PAIR_SEARCH
    * (read-only): 1 LBVH, 2 grid in the last broadphase. */
   B2G_OPT_PAIR_SEARCH = 9,
-  B2G_OPT_LAST_PAIR_SEARCH = 10
+  B2G_OPT_LAST_PAIR_SEARCH = 10,
+  /* How eager steps by colours order their sweeps; the results are the same.
+   * 0 (default): one launch for all velocity iterations and one for all
+   * position iterations, each constraint waiting for its bodies' earlier
+   * updates, where the constraints fit the device at once; else a launch per
+   * colour. 1: always a launch per colour. 2: as 0, with those launches'
+   * workgroups giving up their places (as they do when the device has no room
+   * for all of them), so that one workgroup does all sweeps.
+   * B2G_OPT_LAST_SWEEPS (read-only): 1 a launch per colour, 2 one launch per
+   * phase in the last step by colours. */
+  B2G_OPT_SWEEPS = 11,
+  B2G_OPT_LAST_SWEEPS = 12
 };
 int b2g_set_option(b2g_batch* batch, int32_t option, int32_t value);
 int b2g_get_option(b2g_batch* batch, int32_t option, int32_t* value);

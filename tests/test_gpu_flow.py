@@ -1,0 +1,91 @@
+"""GPU tests of the sweeps ordered by data: one launch runs all velocity
+iterations and one all position iterations, each constraint waiting for its
+bodies' earlier updates (b2g_flow.h). Every body sees the same updates in the
+same order as with a launch per colour, so every state compares bit for bit:
+against a launch per colour (B2G_OPT_SWEEPS 1), and with the launches'
+workgroups made to give up their places, so that one workgroup does all
+sweeps (2).
+"""
+import sys
+
+import numpy as np
+import pytest
+
+from util import GOLDEN, load_pkg, scene_for
+
+pytestmark = pytest.mark.gpu
+S = load_pkg().scenes
+sys.path.insert(0, GOLDEN)
+
+
+def _motors(n=70):
+    """Jointed pairs with limits and motors over a kinematic and a static body, some in contact."""
+    s = S.small_mixed(seed=3, n=20)
+    lift = s.add_body(S.KINEMATIC, 6.0, 2.0, 0.0, 0.3, 0.1, 0.2)
+    s.add_box(lift, 1.5, 0.2)
+    prev = lift
+    for i in range(n):
+        b = s.add_body(S.DYNAMIC, 6.0 + 0.4 * i, 3.0 + 0.02 * (i % 3))
+        s.add_box(b, 0.25, 0.1)
+        s.add_revolute(prev, b, (5.9 + 0.4 * i, 3.0), collide_connected=i % 4 == 0,
+                       limit=(-0.3, 0.4) if i % 3 == 0 else None, motor=(2.0, 30.0) if i % 5 == 0 else None)
+        prev = b if i % 7 else lift if i % 2 else 0
+    return s
+
+
+def _sleepers():
+    import make_golden
+    return make_golden.sleep_scene()
+
+
+CASES = {
+    # scenes, steps, velocity and position iterations, warm starting, sleeping
+    "one_box": ([lambda: S.pyramid(1)], 40, 8, 3, True, False),
+    "pyramid": ([lambda: S.pyramid(20)], 60, 8, 3, True, False),
+    "pyramid_cold": ([lambda: S.pyramid(12)], 30, 8, 3, False, False),
+    "pile": ([lambda: S.random_pile(3001, seed=5, half_w=30.0, height=80.0)], 90, 8, 3, True, False),
+    "chain": ([lambda: scene_for("chain")[0]], 60, 8, 3, True, False),
+    "motors": ([_motors], 90, 8, 3, True, False),
+    "motors_many_iterations": ([_motors], 40, 13, 7, True, False),
+    "motors_no_iterations": ([_motors], 10, 0, 0, True, False),
+    "gas_chains": ([lambda: S.gas_and_chains(4000, 16, 30, seed=0x5C3, half=80.0)], 30, 8, 3, True, False),
+    "worlds_with_joints": ([lambda: S.gas_and_chains(300, 4, 9, seed=1, half=25.0), _motors,
+                            lambda: S.random_pile(200, seed=2, half_w=9.0, height=30.0)], 50, 8, 3, True, False),
+    "sleep": ([_sleepers], 200, 8, 3, True, True),
+    "sleep_joints": ([lambda: S.gas_and_chains(300, 6, 12, seed=7, half=40.0)], 120, 8, 3, True, True),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_gpu_sweeps_ordered_by_data_equal_a_launch_per_colour(engine, name):
+    scenes, steps, vi, pi, warm, sleep = CASES[name]
+    made = [f() for f in scenes]
+    batches = []
+    for mode in (1, 0, 2):
+        b = engine.Batch.from_scenes(made)
+        b.set_option(engine.OPT_SOLVER, engine.SOLVER_COLOURS)
+        b.set_option(engine.OPT_SWEEPS, mode)
+        batches.append(b)
+    ordered = 0
+    for k in range(0, steps, 10):
+        for b in batches:
+            b.advance(10, vi=vi, pi=pi, warm=[warm] * len(made), sleep=[sleep] * len(made))
+        ordered += batches[1].get_option(engine.OPT_LAST_SWEEPS) == 2
+        assert batches[0].get_option(engine.OPT_LAST_SWEEPS) == 1
+        ref = batches[0]
+        for mode, b in ((0, batches[1]), (2, batches[2])):
+            assert np.array_equal(ref.bodies().view(np.uint8), b.bodies().view(np.uint8)), (k, mode, "bodies")
+            assert np.array_equal(ref.contacts().view(np.uint8), b.contacts().view(np.uint8)), (k, mode, "contacts")
+            nj = sum(s.joint_count for s in made)
+            assert np.array_equal(ref.joints(nj).view(np.uint8), b.joints(nj).view(np.uint8)), (k, mode, "joints")
+    assert ordered == steps // 10  # the default did order its sweeps by data
+    for b in batches:
+        b.close()
+
+
+def test_gpu_sweeps_past_the_resident_limit_use_a_launch_per_colour(engine):
+    """More constraints than the launch keeps resident: 512 workgroups of 256 lanes."""
+    sc = S.gas_and_chains(2000, 9000, 15, seed=4, half=700.0)  # 135,000 joints
+    b = engine.Batch.from_scenes([sc]).advance(2)
+    assert b.get_option(engine.OPT_LAST_SWEEPS) == 1
+    b.close()
