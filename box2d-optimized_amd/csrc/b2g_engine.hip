@@ -51,6 +51,7 @@ int dalloc(T** p, size_t n) {
   return B2G_OK;
 }
 
+constexpr size_t kStageBytes = size_t(2) << 20;  // each of a batch's two staging buffers at most
 constexpr int kColourRoundsPerStep = 4;
 // one world: two device-wide rounds, then the one-workgroup finishing pass
 // (k_colour_finish), whose rounds cost a barrier each instead of two launches
@@ -287,6 +288,13 @@ struct b2g_batch {
   int static_shapes = 0;      // shapes of static bodies (their pair segments are sorted every broadphase)
   int tree_ns = -1;           // shape count of the last full build
   bool capturing = false;     // a step graph is being captured: full builds only
+  // pinned staging of body downloads: two chunks, one filled by the device
+  // while the host empties the other
+  void* stage_rec[2] = {nullptr, nullptr};
+  size_t stage_rec_bytes = 0;
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  int stage_room(size_t bytes);
+  int download_records(bool full, int first, int count, void* out);
   void* qbuf = nullptr;       // scratch of the user queries
   size_t qbuf_bytes = 0;
   int query_scratch(size_t bytes);
@@ -359,6 +367,7 @@ int b2g_batch::alloc() {
 #undef A
   d.ccap = NC;
   d.ecap = NC;
+  if ((rc = stage_room(std::min(kStageBytes, sizeof(b2g_body) * (size_t)NB))) != B2G_OK) return rc;
   HIP_TRY(hipHostMalloc((void**)&pinned, 256 * sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&stage_wpar, (size_t)NW * sizeof(float4), hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&stage_wflag, (size_t)NW * sizeof(int), hipHostMallocDefault));
@@ -417,6 +426,10 @@ void b2g_batch::release() {
   graphs_clear();
   if (qbuf) (void)hipFree(qbuf);
   qbuf = nullptr;
+  for (int k = 0; k < 2; ++k) {
+    if (stage_rec[k]) (void)hipHostFree(stage_rec[k]);
+    if (stage_ev[k]) (void)hipEventDestroy(stage_ev[k]);
+  }
   void* ptrs[] = {d.xf, d.pos, d.vel, d.prop, d.prop2, d.force, d.btype, d.bworld, d.wpar, d.wflag, d.wshape0, d.wshape1, d.wbody, d.worder, d.wact, d.wcol, d.wcolmax, d.wfresh,
                   d.wrecolour,
                   d.wbounds, d.wleaf, d.wroot, d.shdr, d.geo, d.smat, d.sfilt, d.aabb, d.joints, d.jsol,
@@ -2321,37 +2334,14 @@ int b2g_get_profile(b2g_batch* b, b2g_profile* out) {
 int b2g_download_bodies(b2g_batch* b, int32_t first, int32_t count, b2g_body* out) {
   if (!b || first < 0 || count < 0 || first + count > b->d.nb) return fail(B2G_ERR_INVALID, "body range");
   if (count == 0) return B2G_OK;
-  std::vector<float4> xf(count), pos(count), vel(count), prop(count), prop2(count), force(count);
-  Dev& d = b->d;
-  hipStream_t st = b->stream;
-  HIP_TRY(hipMemcpyAsync(xf.data(), d.xf + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(pos.data(), d.pos + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(vel.data(), d.vel + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(prop.data(), d.prop + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(prop2.data(), d.prop2 + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(force.data(), d.force + first, count * sizeof(float4), hipMemcpyDeviceToHost, st));
-  std::vector<int> sflag(count);
-  std::vector<float> stime(count);
-  HIP_TRY(hipMemcpyAsync(sflag.data(), d.bsflag + first, count * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipMemcpyAsync(stime.data(), d.bstime + first, count * sizeof(float), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  for (int i = 0; i < count; ++i) {
-    b2g_body& o = out[i];
-    std::memset(&o, 0, sizeof(o));
-    o.type = b->h_btype[first + i];
-    o.world = b->h_bworld[first + i];
-    o.xf[0] = xf[i].x; o.xf[1] = xf[i].y; o.xf[2] = xf[i].z; o.xf[3] = xf[i].w;
-    o.c[0] = pos[i].x; o.c[1] = pos[i].y; o.a = pos[i].z;
-    o.v[0] = vel[i].x; o.v[1] = vel[i].y; o.w = vel[i].z;
-    o.inv_mass = prop[i].x; o.inv_i = prop[i].y;
-    o.local_center[0] = prop[i].z; o.local_center[1] = prop[i].w;
-    o.mass = prop2[i].x; o.gravity_scale = prop2[i].y;
-    o.linear_damping = prop2[i].z; o.angular_damping = prop2[i].w;
-    o.force[0] = force[i].x; o.force[1] = force[i].y; o.torque = force[i].z;
-    o.flags = sflag[i];
-    o.sleep_time = stime[i];
-  }
-  return B2G_OK;
+  static_assert(sizeof(b2g_body) == sizeof(unsigned) * kBodyWords, "k_pack_bodies lays out b2g_body");
+  return b->download_records(true, first, count, out);
+}
+
+int b2g_download_states(b2g_batch* b, int32_t first, int32_t count, float* out) {
+  if (!b || first < 0 || count < 0 || first + count > b->d.nb) return fail(B2G_ERR_INVALID, "body range");
+  if (count == 0) return B2G_OK;
+  return b->download_records(false, first, count, out);
 }
 
 int b2g_download_contacts(b2g_batch* b, int32_t first, int32_t count, b2g_contact* out) {
@@ -2408,6 +2398,51 @@ int b2g_download_contact_colours(b2g_batch* b, int32_t first, int32_t count, int
 }
 
 }  // extern "C"
+
+int b2g_batch::stage_room(size_t bytes) {
+  if (bytes <= stage_rec_bytes) return B2G_OK;
+  const size_t want = std::min(kStageBytes, std::max<size_t>(bytes, 1 << 14));
+  for (int k = 0; k < 2; ++k) {
+    if (stage_rec[k]) (void)hipHostFree(stage_rec[k]);
+    stage_rec[k] = nullptr;
+    stage_rec_bytes = 0;
+    if (!stage_ev[k]) HIP_TRY(hipEventCreateWithFlags(&stage_ev[k], hipEventDisableTiming));
+  }
+  for (int k = 0; k < 2; ++k) HIP_TRY(hipHostMalloc(&stage_rec[k], want, hipHostMallocDefault));
+  stage_rec_bytes = want;
+  return B2G_OK;
+}
+
+// Bodies [first, first + count) as records, chunk by chunk: the device writes
+// a chunk into one staging buffer while the host copies the other out.
+int b2g_batch::download_records(bool full, int first, int count, void* out) {
+  const size_t rec = sizeof(unsigned) * (full ? kBodyWords : kStateWords);
+  int rc = stage_room(std::min(kStageBytes, rec * (size_t)count));
+  if (rc) return rc;
+  const int per = (int)(stage_rec_bytes / rec);
+  int n[2] = {0, 0};
+  for (int at = 0, k = 0, done = 0; done < count; k ^= 1) {
+    if (at < count) {
+      n[k] = std::min(per, count - at);
+      const dim3 grid((n[k] + kBlock - 1) / kBlock);
+      if (full)
+        hipLaunchKernelGGL(k_pack_bodies<true>, grid, dim3(kBlock), 0, stream, d, first + at, n[k],
+                           (unsigned*)stage_rec[k]);
+      else
+        hipLaunchKernelGGL(k_pack_bodies<false>, grid, dim3(kBlock), 0, stream, d, first + at, n[k],
+                           (unsigned*)stage_rec[k]);
+      HIP_TRY(hipEventRecord(stage_ev[k], stream));
+      at += n[k];
+    }
+    const int o = at < count || n[k ^ 1] ? k ^ 1 : k;  // the chunk filled before, if it is not out yet
+    if (n[o] == 0) continue;
+    HIP_TRY(hipEventSynchronize(stage_ev[o]));
+    std::memcpy((char*)out + rec * (size_t)done, stage_rec[o], rec * (size_t)n[o]);
+    done += n[o];
+    n[o] = 0;
+  }
+  return B2G_OK;
+}
 
 int b2g_batch::query_scratch(size_t bytes) {
   if (bytes <= qbuf_bytes) return B2G_OK;

@@ -3424,6 +3424,52 @@ __global__ void k_finish_pairs(Dev d) {
   }
 }
 
+// ---- records for the host -------------------------------------------------
+// Bodies [first, first + count) as the host's records, straight into pinned
+// host memory: a block gathers 256 bodies' fields (16-byte loads), lays the
+// records out in LDS (an odd or 10-word stride: at most two lanes to a bank)
+// and writes them as consecutive words. Bound by the link to the host; eight
+// copies of the field arrays and their assembly on one host core took about 40
+// ms for 1.2M bodies against 14 ms, and 5 ms for a world of 115,000 with its
+// body objects against 0.4 ms.
+// kFull: b2g_body; else centre, angle, velocities and transform (10 floats).
+constexpr int kBodyWords = 25, kStateWords = 10;
+template <bool kFull>
+__global__ void __launch_bounds__(kBlock) k_pack_bodies(Dev d, int first, int count, unsigned* out) {
+  constexpr int W = kFull ? kBodyWords : kStateWords;
+  __shared__ unsigned s_rec[kBlock * W];
+  for (int base = (int)blockIdx.x * kBlock; base < count; base += (int)gridDim.x * kBlock) {
+    const int n = min(kBlock, count - base);
+    if ((int)threadIdx.x < n) {
+      const int b = first + base + (int)threadIdx.x;
+      unsigned* o = s_rec + (int)threadIdx.x * W;
+      auto put = [&](int k, float v) { o[k] = as_uint(v); };
+      const float4 xf = d.xf[b], pos = d.pos[b], vel = d.vel[b];
+      if (kFull) {
+        const float4 prop = d.prop[b], prop2 = d.prop2[b], force = d.force[b];
+        o[0] = (unsigned)d.btype[b];
+        o[1] = (unsigned)d.bworld[b];
+        put(2, xf.x); put(3, xf.y); put(4, xf.z); put(5, xf.w);
+        put(6, pos.x); put(7, pos.y); put(8, pos.z);
+        put(9, prop.z); put(10, prop.w);
+        put(11, vel.x); put(12, vel.y); put(13, vel.z);
+        put(14, prop2.x); put(15, prop.x); put(16, prop.y);
+        put(17, prop2.z); put(18, prop2.w); put(19, prop2.y);
+        put(20, force.x); put(21, force.y); put(22, force.z);
+        o[23] = (unsigned)d.bsflag[b];
+        put(24, d.bstime[b]);
+      } else {
+        put(0, pos.x); put(1, pos.y); put(2, pos.z);
+        put(3, vel.x); put(4, vel.y); put(5, vel.z);
+        put(6, xf.x); put(7, xf.y); put(8, xf.z); put(9, xf.w);
+      }
+    }
+    __syncthreads();
+    for (int k = (int)threadIdx.x; k < n * W; k += kBlock) out[(size_t)base * W + k] = s_rec[k];
+    __syncthreads();
+  }
+}
+
 // ---- standalone narrowphase over caller pairs (b2g_collide_pairs) -----------
 __global__ void __launch_bounds__(kBlock) k_collide_pairs(int n, const int4* __restrict__ ha, const float4* __restrict__ ga,
                                                           const float4* __restrict__ xa, const int4* __restrict__ hb,

@@ -80,7 +80,7 @@ EXPORTS = [
     "b2g_device_count", "b2g_last_error", "b2g_batch_create", "b2g_batch_destroy",
     "b2g_set_worlds", "b2g_set_world_params", "b2g_upload_bodies", "b2g_upload_shapes",
     "b2g_upload_joints", "b2g_upload_contacts", "b2g_batch_step", "b2g_batch_wait",
-    "b2g_get_counts", "b2g_get_profile", "b2g_download_bodies", "b2g_download_contacts",
+    "b2g_get_counts", "b2g_get_profile", "b2g_download_bodies", "b2g_download_states", "b2g_download_contacts",
     "b2g_download_joints", "b2g_download_contact_colours", "b2g_collide_pairs", "b2g_collide_pairs_noalloc",
     "b2g_find_pairs",
     "b2a_world_from_scene", "b2a_world_destroy", "b2a_world_step", "b2a_world_get_bodies",
@@ -138,7 +138,7 @@ def lib():
         L.b2g_set_worlds.argtypes = [_P, _I, _P, _P, _P]
         L.b2g_set_world_params.argtypes = [_P, _I, _I, _P]
         for f in ("b2g_upload_bodies", "b2g_upload_shapes", "b2g_upload_joints",
-                  "b2g_download_bodies", "b2g_download_contacts", "b2g_download_joints",
+                  "b2g_download_bodies", "b2g_download_states", "b2g_download_contacts", "b2g_download_joints",
                   "b2g_download_contact_colours", "b2g_download_solver_points"):
             getattr(L, f).argtypes = [_P, _I, _I, _P]
         L.b2g_upload_contacts.argtypes = [_P, _I, _P]
@@ -392,7 +392,7 @@ class Batch:
     def bodies(self, first=0, count=None):
         if count is None:
             count = self.counts().bodies - first
-        out = np.zeros(count, dtype=BODY_DTYPE)
+        out = np.empty(count, dtype=BODY_DTYPE)
         if count:
             check(self.L.b2g_download_bodies(self.h, first, count, _ptr(out)))
         return out
@@ -520,7 +520,7 @@ class World:
 
     def bodies(self):
         """10 floats per body: centre c (2), angle, v (2), w, transform (p 2, q.s, q.c)."""
-        out = np.zeros((self.nb, 10), dtype=np.float32)
+        out = np.empty((self.nb, 10), dtype=np.float32)
         check(self.L.b2a_world_get_bodies(self.h, _ptr(out)))
         return out
 

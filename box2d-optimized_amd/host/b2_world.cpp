@@ -1446,6 +1446,15 @@ struct b2a_world {
   std::vector<b2Joint*> joints;
 };
 
+// what b2a_world_get_bodies asks of a world beside its public API
+struct b2a_access {
+  // the bodies' states are the device's: no getter has read them since the
+  // last step, and no edit is under way
+  static bool StatesOnDevice(const b2World& w) { return !w.m_bodiesValid && w.m_batch && !w.m_editing; }
+  // a setter changed body i since: its own values hold
+  static bool Edited(const b2World& w, size_t i) { return w.m_dirty[i] != 0; }
+};
+
 // Builds a b2World from a scene description through the public API
 // (CreateBody / CreateFixture / CreateJoint), as user code would.
 static b2a_world* world_from_scene(const b2g_scene* s, int32_t warm_starting) {
@@ -1619,8 +1628,14 @@ int b2a_world_step(b2a_world* w, float dt, int32_t vi, int32_t pi) {
 
 int b2a_world_get_bodies(b2a_world* w, float* out) {
   if (!w) return B2G_ERR_INVALID;
-  for (size_t i = 0; i < w->bodies.size(); ++i) {
+  const size_t n = w->bodies.size();
+  // after a step the states come as one packed read; the b2Body objects are
+  // left for the getters to bring up to date
+  const bool read = n > 0 && b2a_access::StatesOnDevice(*w->world) &&
+                    b2g_download_states(w->world->GetDeviceBatch(), 0, (int32_t)n, out) == B2G_OK;
+  for (size_t i = 0; i < n; ++i) {
     b2Body* b = w->bodies[i];
+    if (read && !b2a_access::Edited(*w->world, i)) continue;
     const b2Vec2 c = b->GetWorldCenter();
     const b2Vec2 v = b->GetLinearVelocity();
     const b2Transform& xf = b->GetTransform();

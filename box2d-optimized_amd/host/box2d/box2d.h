@@ -684,6 +684,7 @@ class b2World {
   static void FixtureToRecord(const b2Fixture* f, b2g_shape* out);
   static void JointToRecord(const b2Joint* j, b2g_revolute* out);
   void SyncBodies() const;
+  friend struct b2a_access;
   void SyncContacts();
   void ContactFromRecord(const b2g_contact& r, b2Contact* c) const;
   void SyncJoints() const;

@@ -337,6 +337,8 @@ int b2g_get_option(b2g_batch* batch, int32_t option, int32_t* value);
 int b2g_kernel_time(b2g_batch* batch, double* total_ms, int64_t* launches, int64_t* items);
 int b2g_get_profile(b2g_batch* batch, b2g_profile* out);
 int b2g_download_bodies(b2g_batch* batch, int32_t first, int32_t count, b2g_body* out);
+/* 10 floats per body: centre c (2), angle, v (2), w, transform (p 2, q.s, q.c) */
+int b2g_download_states(b2g_batch* batch, int32_t first, int32_t count, float* out);
 /* contacts are ordered by (min shape, max shape); out may be NULL to query the count */
 int b2g_download_contacts(b2g_batch* batch, int32_t first, int32_t count, b2g_contact* out);
 int b2g_download_joints(b2g_batch* batch, int32_t first, int32_t count, b2g_revolute* out);
