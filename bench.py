@@ -153,8 +153,7 @@ def batched_section(pkg, worlds: int, warmup: int, steps: int, sample_every: int
     batch, stepped one after another with a host sync per step, as a caller
     looping over b2World::Step would) on a sample of the same worlds, and with
     the reference CPU Step on the same sample. The warm-up is at least 12
-    steps: the per-world solver's workgroup autotuner takes the first 10
-    (eager steps, whatever the launch mode)."""
+    steps (the first ones size the buffers)."""
     import numpy as np
     S, eng = pkg.scenes, pkg.engine
     warmup = max(warmup, 12)

@@ -22,6 +22,7 @@
 #include "b2g_grid.h"
 #include "b2g_partition.h"
 #include "b2g_flow.h"
+#include "b2g_worlds.h"
 
 using namespace b2g;
 
@@ -51,6 +52,8 @@ int dalloc(T** p, size_t n) {
   return B2G_OK;
 }
 
+// the largest class a single world's solve takes
+constexpr int kOneWorldClass = kPairClass;
 constexpr size_t kStageBytes = size_t(2) << 20;  // each of a batch's two staging buffers at most
 constexpr int kColourRoundsPerStep = 4;
 // one world: two device-wide rounds, then the one-workgroup finishing pass
@@ -220,12 +223,9 @@ struct b2g_batch {
       if (h_params[w].active && h_params[w].allow_sleep) return true;
     return false;
   }
-  int world_block = 0;       // threads per world workgroup (0: autotune)
-  int tuned_block = 0;       // chosen by the autotuner (or world_block)
-  bool tuned_lds = false;    // autotuner: stage world bodies in LDS
-  int world_lds = -1;        // -1 autotune, 0 off, 1 on (when the worlds fit)
-  int tune_step = 0;         // autotuner progress: two timed steps per candidate
-  float tune_ms[16] = {};
+  int world_block = 0;       // B2G_OPT_WORLD_BLOCK (0: the classes of b2g_worlds.h)
+  int world_lds = -1;        // B2G_OPT_WORLD_LDS
+  int class_count[kWorldClasses] = {};  // worlds per class, as the step read them
   int last_path = 0;         // 1 colour-major sweeps, 2 per-world, 3 cells
 
   int alloc();
@@ -265,6 +265,9 @@ struct b2g_batch {
   int world_block_now() const;
   bool world_lds_now() const;
   void launch_solve_worlds(int vi, int pi);
+  bool use_classes() const;
+  bool one_world_launch() const;
+  void launch_classes(int vi, int pi);
   int eager_step(int vi, int pi, unsigned flags);
   int graph_step(int vi, int pi, unsigned flags);
   int scan(const int* in, const int* n_dev, int n_host, int* out, int* total, long long n_bound);
@@ -311,7 +314,7 @@ int b2g_batch::alloc() {
   if ((rc = dalloc(&(ptr), (size_t)(n))) != B2G_OK) return rc
   A(d.xf, NB); A(d.pos, NB); A(d.vel, NB); A(d.prop, NB); A(d.prop2, NB); A(d.force, NB);
   A(d.btype, NB); A(d.bworld, NB);
-  A(d.wpar, NW); A(d.wflag, NW); A(d.wsort, NW); A(d.wshape0, NW); A(d.wshape1, NW); A(d.wbody, NW); A(d.worder, NW); A(d.wact, NW);
+  A(d.wpar, NW); A(d.wflag, NW); A(d.wsort, NW); A(d.wshape0, NW); A(d.wshape1, NW); A(d.wbody, NW); A(d.worder, NW); A(d.wact, NW); A(d.wclass, (size_t)kWorldClasses * NW);
   A(d.wcol, (size_t)NW * (kColourSlots + 1));
   A(d.wcolmax, NW); A(d.wfresh, NW); A(d.wrecolour, NW); A(d.wbounds, 4 * NW); A(d.wleaf, 2 * NW); A(d.wroot, NW);
   A(d.shdr, NS); A(d.geo, 9 * (size_t)NS); A(d.smat, NS); A(d.sfilt, NS); A(d.aabb, NS);
@@ -430,7 +433,7 @@ void b2g_batch::release() {
     if (stage_rec[k]) (void)hipHostFree(stage_rec[k]);
     if (stage_ev[k]) (void)hipEventDestroy(stage_ev[k]);
   }
-  void* ptrs[] = {d.xf, d.pos, d.vel, d.prop, d.prop2, d.force, d.btype, d.bworld, d.wpar, d.wflag, d.wshape0, d.wshape1, d.wbody, d.worder, d.wact, d.wcol, d.wcolmax, d.wfresh,
+  void* ptrs[] = {d.xf, d.pos, d.vel, d.prop, d.prop2, d.force, d.btype, d.bworld, d.wpar, d.wflag, d.wshape0, d.wshape1, d.wbody, d.worder, d.wact, d.wclass, d.wcol, d.wcolmax, d.wfresh,
                   d.wrecolour,
                   d.wbounds, d.wleaf, d.wroot, d.shdr, d.geo, d.smat, d.sfilt, d.aabb, d.joints, d.jsol,
                   d.jorder, d.wj_off, d.wj_list, d.jisland, d.bj_off, d.bj_other, d.ckey, d.cpair, d.cman, d.cmat, d.ccol,
@@ -1106,11 +1109,11 @@ void b2g_batch::enqueue_islands_and_init() {
   if (worlds_contiguous && max_world_bodies <= kIslandLdsLarge) {
     // one workgroup per world, the forest in LDS
     if (max_world_bodies <= kIslandLdsSmall)
-      hipLaunchKernelGGL(k_world_islands<kIslandLdsSmall>, dim3(d.nw), dim3(256), 0, is, d);
+      hipLaunchKernelGGL(k_world_islands<kIslandLdsSmall>, dim3(d.nw), dim3(256), 0, is, d, d.worder);
     else if (max_world_bodies <= kIslandLdsMid)
-      hipLaunchKernelGGL(k_world_islands<kIslandLdsMid>, dim3(d.nw), dim3(512), 0, is, d);
+      hipLaunchKernelGGL(k_world_islands<kIslandLdsMid>, dim3(d.nw), dim3(512), 0, is, d, d.worder);
     else
-      hipLaunchKernelGGL(k_world_islands<kIslandLdsLarge>, dim3(d.nw), dim3(1024), 0, is, d);
+      hipLaunchKernelGGL(k_world_islands<kIslandLdsLarge>, dim3(d.nw), dim3(1024), 0, is, d, d.worder);
   } else {
     hipLaunchKernelGGL(k_island_link, dim3(grid_for(std::max(est_cons, 1) + d.nj)), dim3(kBlock), 0, is, d);
     hipLaunchKernelGGL(k_island_label, dim3(grid_for(d.nb)), dim3(kBlock), 0, is, d);
@@ -1394,31 +1397,87 @@ bool b2g_batch::use_per_world() const {
   return d.nw >= 2 && max_world_bodies <= 8192;
 }
 
-// autotuner candidates: workgroup size x bodies staged in LDS or not (one
-// timed step each); a launch's stage holds up to 156 KB of bodies (a gfx950
-// workgroup may take 160 KB of LDS, the whole CU's: every world the
-// per-world solver takes, 8192 bodies at most, fits)
-static const int kWorldBlocks[] = {64, 128, 256, 512, 1024};
-constexpr int kWorldBlockCount = 5;
+// a launch's LDS stage holds up to 156 KB of bodies (a gfx950 workgroup may
+// take 160 KB of LDS, the whole CU's: every world the per-world solver takes,
+// 8192 bodies at most, fits)
 constexpr int kLdsBodyLimit = (156 * 1024) / 16;
 constexpr int kSmallWorldLds = 512;
+constexpr int kWorldBlockDefault = 256;
 
-int b2g_batch::world_block_now() const {
-  if (world_block > 0) return world_block;
-  if (tuned_block > 0) return tuned_block;
-  return kWorldBlocks[std::min(tune_step, 2 * kWorldBlockCount - 1) % kWorldBlockCount];
+int b2g_batch::world_block_now() const { return world_block > 0 ? world_block : kWorldBlockDefault; }
+
+// (workgroups of 64 to 512 with and without the bodies in LDS, captured steps
+// of settled worlds: 1000 worlds of a few to hundreds of bodies take 0.90 ms at
+// 256 with the stage, 1.00 without, 1.02 and 1.03 at 128; 4096 equal ones 3.60
+// and 3.78, 3.54 and 3.94 at 128; 64 large ones 0.43 and 0.45, 0.51 and 0.54. A
+// world past a launch's stage reads its bodies from global memory)
+bool b2g_batch::world_lds_now() const { return world_lds > 0 || (world_lds < 0 && world_block == 0); }
+
+// The per-world solver by classes (b2g_worlds.h), unless the caller picked a
+// workgroup size or stage for k_solve_worlds.
+bool b2g_batch::use_classes() const {
+  return use_per_world() && world_block == 0 && world_lds < 0 && max_world_bodies <= kIslandLdsMid;
 }
 
-bool b2g_batch::world_lds_now() const {
-  if (world_lds == 0) return false;  // (a world past a launch's stage reads its bodies from global memory)
-  if (world_lds > 0) return true;
-  if (world_block > 0 || tuned_block > 0) return tuned_lds;
-  return std::min(tune_step, 2 * kWorldBlockCount - 1) >= kWorldBlockCount;
+// One joint-free world whose solve fits a workgroup of b2g_worlds.h, going by
+// the last step's constraints (the step checks its own): a 20-row pyramid's
+// step with its read-back takes 186 us, with the flow launches 269. Past the
+// largest class the flow launches spread over the device.
+bool b2g_batch::one_world_launch() const {
+  return solver_mode == B2G_SOLVER_AUTO && d.nw == 1 && per_world_ok && !d.sleep_on && world_block == 0 &&
+         world_lds < 0 && sweeps == 0 && max_world_bodies <= class_bodies(kOneWorldClass) &&
+         est_cons <= class_slots(kOneWorldClass);
+}
+
+// Every active world's solve: one launch for the classes and, beside it on
+// the side stream, the largest worlds. Sized by the class counts the step has
+// read, so captured steps keep k_solve_worlds (a graph also replays its
+// branches one after the other: 1000 worlds, a replayed step 1.2 ms against
+// 1.1).
+void b2g_batch::launch_classes(int vi, int pi) {
+  tbegin(B2G_KERNEL_SOLVER);
+  const int rounds = rounds_pending;
+  round_host += (unsigned)rounds_pending;
+  rounds_pending = 0;
+  const int last = kWorldClasses - 1;
+  int top = 0;  // one world: a workgroup of its class's size
+  for (int c = 0; c < kPairClass; ++c)
+    if (class_count[c] > 0) top = c;
+  const int threads = d.nw == 1 ? (class_slots(top) + kWave - 1) / kWave * kWave : kGroupThreads;
+  int blocks = 0;
+  for (int c = 0; c < kPairClass; ++c) blocks += class_blocks(class_count[c], c, threads == kGroupThreads);
+  const int pairs = class_count[kPairClass], over = class_count[last];
+  // the largest worlds first, on the side stream beside the others
+  const bool fork = over + pairs > 0 && blocks > 0;
+  hipStream_t st = fork ? side : stream;
+  if (fork) {
+    (void)hipEventRecord(fork_ev, stream);
+    (void)hipStreamWaitEvent(side, fork_ev, 0);
+  }
+  if (over > 0) {
+    const int* list = d.wclass + (size_t)last * d.nw;
+    hipLaunchKernelGGL(k_world_colour_sort, dim3(over), dim3(kBlock), 0, st, d, 0, list);
+    hipLaunchKernelGGL(k_world_islands<kIslandLdsMid>, dim3(over), dim3(512), 0, st, d, list);
+    hipLaunchKernelGGL(k_worlds_init, dim3(over, 16), dim3(kBlock), 0, st, d, list);
+    const int bodies = std::min(max_world_bodies, kLdsBodyLimit);
+    hipLaunchKernelGGL(k_solve_worlds<true>, dim3(over), dim3(1024), sizeof(float4) * (size_t)bodies, st, d, vi, pi,
+                       0, list, bodies);
+  }
+  if (pairs > 0)
+    hipLaunchKernelGGL((k_step_worlds<kPairThreads, kGroupSlots / kPairThreads>), dim3(pairs), dim3(kPairThreads), 0, st,
+                       d, vi, pi, blocks > 0 ? 0 : rounds, kPairClass, kPairClass);
+  if (fork) (void)hipEventRecord(join_ev, side);
+  // (with no world in any class the launch still moves the claim-round base on)
+  if (blocks > 0 || pairs <= 0)
+    hipLaunchKernelGGL((k_step_worlds<kGroupThreads, 1>), dim3(std::max(blocks, 1)), dim3(threads), 0, stream, d, vi,
+                       pi, rounds, 0, kPairClass - 1);
+  if (fork) (void)hipStreamWaitEvent(stream, join_ev, 0);
+  tend(B2G_KERNEL_SOLVER, est_cons);
 }
 
 // Worlds of more than kBigWorldBodies bodies (the first ones in worder) get
 // full 1024-thread workgroups in a launch of their own, beside the launch of
-// the other worlds at the tuned workgroup size (on the side stream): one
+// the other worlds at world_block_now() threads (on the side stream): one
 // large world on a small workgroup would otherwise set the whole batch's
 // solve time. Every world runs the same kernel either way.
 
@@ -1503,8 +1562,7 @@ int b2g_batch::step(int vi, int pi, unsigned flags) {
   const bool prof_on = (flags & B2G_STEP_PROFILE) != 0;
   const bool graph_ok = (flags & B2G_STEP_GRAPH) && !prof_on && timed_kernel < 0 && !d.sleep_on &&
                         !(flags & B2G_STEP_FIND_NEW_CONTACTS) &&
-                        (graph_K > 0 || use_cells()) &&  // a cells step needs no colour count from an eager one
-                        (!use_per_world() || world_block > 0 || tuned_block > 0);
+                        (graph_K > 0 || use_cells());  // a cells step needs no colour count from an eager one
   if (graph_ok) return graph_step(vi, pi, flags);
   return eager_step(vi, pi, flags);
 }
@@ -1614,48 +1672,42 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
   // the contact list is the last broadphase's pair list: world contact
   // ranges are segment offsets
   d.segs = pairs_current && worlds_contiguous ? 1 : 0;
+  const bool one = one_world_launch();
+  const bool classes = use_classes() || one;
+  d.classes_on = classes ? 1 : 0;
   if (!use_per_world()) use_flow();
   enqueue_collide_and_colour_eager();
+  d.classes_on = 0;
   if (prof_on) HIP_TRY(hipEventRecord(ev[1], stream));
   int rc;
-  if (use_per_world()) {
-    last_path = 2;
+  bool per_world = use_per_world();
+  if (classes || per_world) {
     if ((rc = read_counters())) return rc;
     if ((rc = status_error())) return rc;  // an earlier (asynchronous) step overflowed
-    const int pw_colours = pinned[C_NCOLOURS];  // last step's (normal colours are what it reports)
+    for (int c = 0; c < kWorldClasses; ++c) class_count[c] = pinned[kCntClass + c];
+    est_cons = pinned[C_CONS];
+    // (the world outgrew the classes: the colour sweeps below)
+    if (one) per_world = est_cons <= class_slots(kOneWorldClass) && class_count[kWorldClasses - 1] == 0;
+  }
+  if (per_world) {
+    last_path = 2;
     for (int extra = 0; pinned[C_REMAIN] > 0; extra += 2) {  // colour everything first
       if (extra > 4096) return fail(B2G_ERR_CAPACITY, "colouring did not converge");
       enqueue_colour_round(kMaxColours);
       enqueue_colour_round(kMaxColours);
       if ((rc = read_counters())) return rc;
     }
-    est_cons = pinned[C_CONS];
-    hipLaunchKernelGGL(k_world_colour_sort, dim3(d.nw), dim3(kBlock), 0, stream, d, rounds_pending);
-    round_host += (unsigned)rounds_pending;
-    rounds_pending = 0;
-    enqueue_islands_and_init();
-    enqueue_islands_join();
-    const bool tuning = world_block == 0 && tuned_block == 0;
-    if (tuning) HIP_TRY(hipEventRecord(ev[5], stream));
-    launch_solve_worlds(vi, pi);
-    if (tuning) {
-      HIP_TRY(hipEventRecord(ev[6], stream));
-      HIP_TRY(hipEventSynchronize(ev[6]));
-      float ms = 0.0f;
-      HIP_TRY(hipEventElapsedTime(&ms, ev[5], ev[6]));
-      const bool lds_ok = world_lds != 0;
-      const int ncand = lds_ok ? 2 * kWorldBlockCount : kWorldBlockCount;
-      tune_ms[tune_step] = ms;
-      if (++tune_step >= ncand) {
-        int best = 0;
-        for (int c = 1; c < ncand; ++c)
-          if (tune_ms[c] < tune_ms[best]) best = c;
-        tuned_block = kWorldBlocks[best % kWorldBlockCount];
-        tuned_lds = best >= kWorldBlockCount;
-      }
+    if (classes) {
+      launch_classes(vi, pi);
+    } else {
+      hipLaunchKernelGGL(k_world_colour_sort, dim3(d.nw), dim3(kBlock), 0, stream, d, rounds_pending, d.worder);
+      round_host += (unsigned)rounds_pending;
+      rounds_pending = 0;
+      enqueue_islands_and_init();
+      enqueue_islands_join();
+      launch_solve_worlds(vi, pi);
     }
     graph_K = kMaxColours;
-    (void)pw_colours;
     if (prof_on) HIP_TRY(hipEventRecord(ev[2], stream));
     if (!(flags & B2G_STEP_SKIP_BROADPHASE)) {
       if ((rc = broadphase(false))) return rc;
@@ -1767,7 +1819,7 @@ int b2g_batch::enqueue_graph_body(int vi, int pi, unsigned flags, int K) {
   hipLaunchKernelGGL(k_colour_leftover, dim3(grid_for(std::max(est_cons, 256) * 5 / 4)), dim3(kBlock), 0, stream,
                      d);
   if (use_per_world()) {
-    hipLaunchKernelGGL(k_world_colour_sort, dim3(d.nw), dim3(kBlock), 0, stream, d, rounds_pending);
+    hipLaunchKernelGGL(k_world_colour_sort, dim3(d.nw), dim3(kBlock), 0, stream, d, rounds_pending, d.worder);
     round_host += (unsigned)rounds_pending;
     rounds_pending = 0;
     enqueue_islands_and_init();
@@ -2246,18 +2298,14 @@ int b2g_set_option(b2g_batch* b, int32_t option, int32_t value) {
       b->solver_mode = value;
       break;
     case B2G_OPT_WORLD_LDS:
-      if (value < -1 || value > 1) return fail(B2G_ERR_INVALID, "world LDS staging: -1 (autotune), 0 or 1");
+      if (value < -1 || value > 1) return fail(B2G_ERR_INVALID, "world LDS staging: -1 (the engine's choice), 0 or 1");
       b->world_lds = value;
-      b->tuned_block = 0;
-      b->tune_step = 0;
       break;
     case B2G_OPT_WORLD_BLOCK:
       if (value != 0 && (value < 64 || value > 1024 || (value & 63))) {
-        return fail(B2G_ERR_INVALID, "world block: 0 (autotune) or a multiple of 64 in [64, 1024]");
+        return fail(B2G_ERR_INVALID, "world block: 0 (the engine's choice) or a multiple of 64 in [64, 1024]");
       }
       b->world_block = value;
-      b->tuned_block = 0;
-      b->tune_step = 0;
       break;
     case B2G_OPT_KEEP_IDLE:
       if (value < 0 || value > 1) return fail(B2G_ERR_INVALID, "keep idle: 0 or 1");
@@ -2291,7 +2339,7 @@ int b2g_get_option(b2g_batch* b, int32_t option, int32_t* value) {
   switch (option) {
     case B2G_OPT_SOLVER: *value = b->solver_mode; break;
     case B2G_OPT_WORLD_BLOCK: *value = b->world_block; break;
-    case B2G_OPT_TUNED_WORLD_BLOCK: *value = b->world_block > 0 ? b->world_block : b->tuned_block; break;
+    case B2G_OPT_TUNED_WORLD_BLOCK: *value = b->world_block_now(); break;
     case B2G_OPT_LAST_SOLVER: *value = b->last_path; break;
     case B2G_OPT_PER_WORLD_ELIGIBLE: *value = b->per_world_ok ? 1 : 0; break;
     case B2G_OPT_WORLD_LDS: *value = b->world_lds; break;

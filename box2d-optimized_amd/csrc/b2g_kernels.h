@@ -66,6 +66,24 @@ constexpr int kCntColOff = 32;  // the colour offsets sit this many ints into th
 
 // all device arrays, passed by value to every kernel
 constexpr int kFlowCtl = 64;
+// A world's class says how many worlds of its size share a workgroup of the
+// one-launch solver (b2g_worlds.h): the most whose even share of its 1024
+// contact slots holds the world's solved contacts, and of its 2048 bodies the
+// world's bodies. The last but one class holds one world of up to 2048
+// contacts and 4096 bodies, the last the worlds past that.
+constexpr int kGroupThreads = 1024, kGroupSlots = 2048, kGroupBodies = 4096;
+constexpr int kWorldClasses = 13;
+constexpr int kCntClass = 16;  // cnt[16 + class]: worlds in each class's list
+constexpr int kPairClass = kWorldClasses - 2;  // one world, two or more contacts to a lane
+__device__ __host__ __forceinline__ constexpr int class_worlds(int c) {  // 16, 12, 10, 8, 7 .. 1, 1
+  return c == 0 ? 16 : c == 1 ? 12 : c == 2 ? 10 : c == kPairClass ? 1 : 11 - c;
+}
+__device__ __host__ __forceinline__ constexpr int class_slots(int c) {
+  return c == kPairClass ? kGroupSlots : kGroupThreads / class_worlds(c);
+}
+__device__ __host__ __forceinline__ constexpr int class_bodies(int c) {
+  return c == kPairClass ? kGroupBodies : kGroupBodies / 2 / class_worlds(c);
+}
 // bytes from one body's flow state to the next: a cache line each (16 bytes,
 // eight bodies to a line: 322 us per velocity phase of a settled pile of
 // 20,000 against 242)
@@ -89,6 +107,8 @@ struct Dev {
   int2* wbody;    // body range of each world (worlds laid out world after world)
   int* worder;    // worlds by decreasing size: the per-world solver's block order
   int* wact;      // the worlds active in the step, in the same order (mostly idle batches)
+  int classes_on; // this step lists the active worlds by class (b2g_worlds.h)
+  int* wclass;    // kWorldClasses lists of nw: the active worlds of each class
   int* wcol;      // per world: kColourSlots + 1 slot offsets of its colour groups
   int* wcolmax;   // per world: highest normal colour used this step (-1: none)
   int* wfresh;    // per world: colours of its last colouring from scratch (0: none yet)
@@ -326,6 +346,7 @@ __global__ void k_events_reset(Dev d) {
 __device__ __forceinline__ void reset_colour_counters(const Dev& d) {
   for (int c = threadIdx.x; c < kColourSlots; c += blockDim.x) d.col_count[c] = 0;
   if (threadIdx.x < kFlowCtl) d.flow_ctl[threadIdx.x] = 0;
+  if (threadIdx.x < kWorldClasses) d.cnt[kCntClass + threadIdx.x] = 0;
   if (threadIdx.x == 0) {
     d.cnt[C_REMAIN] = 0;
     d.cnt[C_PENDING] = 0;
@@ -571,10 +592,24 @@ __global__ void __launch_bounds__(kBlock) k_touch_scan_apply(Dev d, const int* _
 // ===========================================================================
 __device__ __forceinline__ bool is_dyn(const Dev& d, int b) { return d.btype[b] == kDynamicBody; }
 
+// the solved contacts of world w in the compacted list, [first, end)
+__device__ __forceinline__ int2 world_solved(const Dev& d, int w);
+
 // Contacts that stay touching keep last step's colour if it is below the
-// colour limit `K` of this step; the rest are coloured by claim rounds.
+// colour limit `K` of this step; the rest are coloured by claim rounds. The
+// same launch lists the active worlds by class.
 __global__ void __launch_bounds__(kBlock) k_colour_init(Dev d, int K) {
   const int n = d.cnt[C_CONS];
+  if (d.classes_on) {
+    B2G_FOR(w, 0, d.nw) {
+      if (!world_active(d, w)) continue;
+      const int2 t = world_solved(d, w);
+      const int nb = d.wbody[w].y - d.wbody[w].x;
+      int c = 0;
+      while (c < kWorldClasses - 1 && (t.y - t.x > class_slots(c) || nb > class_bodies(c))) ++c;
+      d.wclass[(size_t)c * d.nw + atomicAdd(&d.cnt[kCntClass + c], 1)] = w;
+    }
+  }
   B2G_FOR(k, 0, n) {
     const int c = d.clist[k];
     const int2 bp = d.cbody[k];  // the bodies, without the contact -> shape -> body chain
@@ -958,6 +993,12 @@ __device__ __forceinline__ int2 world_contacts(const Dev& d, int w) {
                    lower_bound_u64(d.ckey, nc, (uint64_t)(uint32_t)s1 << 32));
 }
 
+__device__ __forceinline__ int2 world_solved(const Dev& d, int w) {
+  const int nc = d.cnt[C_CONTACTS], total = d.cnt[C_CONS];
+  const int2 cr = world_contacts(d, w);
+  return make_int2(cr.x < nc ? d.tpos[cr.x] : total, cr.y < nc ? d.tpos[cr.y] : total);
+}
+
 // Islands of one world per workgroup, with the union-find forest in LDS
 // (kCap >= the world's body count). Same forest rule as k_island_link (the
 // larger root hooks under the smaller), so every island is labelled by its
@@ -987,19 +1028,19 @@ __device__ __forceinline__ void lds_union(int* par, int a, int b) {
   }
 }
 
+// The worlds of `order`, one per workgroup.
 template <int kCap>
-__global__ void __launch_bounds__(1024) k_world_islands(Dev d) {
+__global__ void __launch_bounds__(1024) k_world_islands(Dev d, const int* order) {
   __shared__ int par[kCap];
   __shared__ int range[2];
-  const int w = d.worder[blockIdx.x];
+  const int w = order[blockIdx.x];
   if (!world_active(d, w)) return;  // the whole workgroup leaves
   const int2 wb = d.wbody[w];
   const int b0 = wb.x, nbw = wb.y - wb.x;
   if (threadIdx.x == 0) {
-    const int nc = d.cnt[C_CONTACTS], total = d.cnt[C_CONS];
-    const int2 cr = world_contacts(d, w);
-    range[0] = cr.x < nc ? d.tpos[cr.x] : total;
-    range[1] = cr.y < nc ? d.tpos[cr.y] : total;
+    const int2 t = world_solved(d, w);
+    range[0] = t.x;
+    range[1] = t.y;
   }
   for (int i = threadIdx.x; i < nbw; i += blockDim.x) par[i] = i;
   __syncthreads();
@@ -1109,160 +1150,175 @@ __device__ __forceinline__ void island_assign(const Dev& d, int n, int k) {
 //   pc0 localPoint localNormal  pc1 localPoints[0..1]  pc2 localCenterA/B
 //   pc3 mA mB iA iB             pc4 radiusA radiusB type pointCount
 // ===========================================================================
+// One solved contact's constraint: fields vc 0 .. 9 and pc 0 .. 4.
+struct ConFields {
+  float4 v[10], p[5];
+};
+// Contact c of shapes pr on bodies ia, ib of world w, whose states are given.
+__device__ __forceinline__ ConFields contact_fields(const Dev& d, int c, int2 pr, int ia, int ib, int w, float4 posA,
+                                                    float4 posB, float4 velA, float4 velB) {
+  const float4 pa = d.prop[ia], pb = d.prop[ib];
+  const float mA = pa.x, iA = pa.y, mB = pb.x, iB = pb.y;
+  const vec2 lcA = mk(pa.z, pa.w), lcB = mk(pb.z, pb.w);
+  const float4 m0 = d.cman[4 * (size_t)c + 0], m1 = d.cman[4 * (size_t)c + 1];
+  const float4 m2 = d.cman[4 * (size_t)c + 2], m3 = d.cman[4 * (size_t)c + 3];
+  const int mtype = as_int(m3.z) & 0xff;
+  const int count = (as_int(m3.z) >> 8) & 0xff;
+  const float4 mat = d.cmat[c];
+  const float rA = d.geo[9 * (size_t)pr.x].x, rB = d.geo[9 * (size_t)pr.y].x;
+  const float4 wp = d.wpar[w];
+  const bool warm = (d.wflag[w] & 1) != 0;
+  const float ratio = wp.w;
+
+  float ni0 = 0.0f, ti0 = 0.0f, ni1 = 0.0f, ti1 = 0.0f;
+  if (warm) {
+    ni0 = ratio * m0.z;
+    ti0 = ratio * m0.w;
+    ni1 = ratio * m1.z;
+    ti1 = ratio * m1.w;
+  }
+  const vec2 cA = mk(posA.x, posA.y), cB = mk(posB.x, posB.y);
+  const vec2 vA = mk(velA.x, velA.y), vB = mk(velB.x, velB.y);
+  const float wA = velA.z, wB = velB.z;
+  xform xfA, xfB;
+  xfA.q = rot_of(posA.z);
+  xfB.q = rot_of(posB.z);
+  xfA.p = cA - mul(xfA.q, lcA);
+  xfB.p = cB - mul(xfB.q, lcB);
+  // b2WorldManifold::Initialize (src/collision/b2_collision.cpp:26-90)
+  vec2 normal, wp0 = mk(0.0f, 0.0f), wp1 = mk(0.0f, 0.0f);
+  const vec2 ln = mk(m2.x, m2.y), lp = mk(m2.z, m2.w);
+  const vec2 lp0 = mk(m0.x, m0.y), lp1 = mk(m1.x, m1.y);
+  if (mtype == kManCircles) {
+    normal = mk(1.0f, 0.0f);
+    const vec2 pA = mul(xfA, lp);
+    const vec2 pB = mul(xfB, lp0);
+    if (dist_sq(pA, pB) > kEpsilon * kEpsilon) normal = normalize(pB - pA);
+    const vec2 qA = pA + rA * normal;
+    const vec2 qB = pB - rB * normal;
+    wp0 = 0.5f * (qA + qB);
+  } else if (mtype == kManFaceA) {
+    normal = mul(xfA.q, ln);
+    const vec2 plane = mul(xfA, lp);
+    {
+      const vec2 clip = mul(xfB, lp0);
+      const vec2 qA = clip + (rA - dot(clip - plane, normal)) * normal;
+      const vec2 qB = clip - rB * normal;
+      wp0 = 0.5f * (qA + qB);
+    }
+    if (count > 1) {
+      const vec2 clip = mul(xfB, lp1);
+      const vec2 qA = clip + (rA - dot(clip - plane, normal)) * normal;
+      const vec2 qB = clip - rB * normal;
+      wp1 = 0.5f * (qA + qB);
+    }
+  } else {
+    normal = mul(xfB.q, ln);
+    const vec2 plane = mul(xfB, lp);
+    {
+      const vec2 clip = mul(xfA, lp0);
+      const vec2 qB = clip + (rB - dot(clip - plane, normal)) * normal;
+      const vec2 qA = clip - rA * normal;
+      wp0 = 0.5f * (qA + qB);
+    }
+    if (count > 1) {
+      const vec2 clip = mul(xfA, lp1);
+      const vec2 qB = clip + (rB - dot(clip - plane, normal)) * normal;
+      const vec2 qA = clip - rA * normal;
+      wp1 = 0.5f * (qA + qB);
+    }
+    normal = -normal;
+  }
+  const vec2 tangent = cross(normal, 1.0f);
+  vec2 rA0 = wp0 - cA, rB0 = wp0 - cB, rA1 = wp1 - cA, rB1 = wp1 - cB;
+  float nm0, tm0, bias0 = 0.0f, nm1 = 0.0f, tm1 = 0.0f, bias1 = 0.0f;
+  {
+    const float rnA = cross(rA0, normal), rnB = cross(rB0, normal);
+    const float kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
+    nm0 = kn > 0.0f ? 1.0f / kn : 0.0f;
+    const float rtA = cross(rA0, tangent), rtB = cross(rB0, tangent);
+    const float kt = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
+    tm0 = kt > 0.0f ? 1.0f / kt : 0.0f;
+    const float vrel = dot(normal, vB + cross(wB, rB0) - (vA + cross(wA, rA0)));
+    if (vrel < -mat.z) bias0 = -mat.y * vrel;
+  }
+  if (count > 1) {
+    const float rnA = cross(rA1, normal), rnB = cross(rB1, normal);
+    const float kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
+    nm1 = kn > 0.0f ? 1.0f / kn : 0.0f;
+    const float rtA = cross(rA1, tangent), rtB = cross(rB1, tangent);
+    const float kt = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
+    tm1 = kt > 0.0f ? 1.0f / kt : 0.0f;
+    const float vrel = dot(normal, vB + cross(wB, rB1) - (vA + cross(wA, rA1)));
+    if (vrel < -mat.z) bias1 = -mat.y * vrel;
+  }
+  int vcount = count, pcount = count;
+  if (d.sleep_on) {  // a sleeping island is not built (b2_world.cpp:535-539): no points to solve
+    const int isl = d.btype[ia] != kStaticBody ? d.parent[ia] : d.parent[ib];
+    if (d.isl_awake[isl]) d.isl_cons[isl] = 1;
+    else vcount = pcount = 0;
+  }
+  mat22 K = {mk(0.0f, 0.0f), mk(0.0f, 0.0f)}, NM = K;
+  if (count == 2 && vcount == 2) {  // block solver preparation (:236-256)
+    const float rn1A = cross(rA0, normal), rn1B = cross(rB0, normal);
+    const float rn2A = cross(rA1, normal), rn2B = cross(rB1, normal);
+    const float k11 = mA + mB + iA * rn1A * rn1A + iB * rn1B * rn1B;
+    const float k22 = mA + mB + iA * rn2A * rn2A + iB * rn2B * rn2B;
+    const float k12 = mA + mB + iA * rn1A * rn2A + iB * rn1B * rn2B;
+    const float kMaxCond = 1000.0f;
+    if (k11 * k11 < kMaxCond * (k11 * k22 - k12 * k12)) {
+      K.ex = mk(k11, k12);
+      K.ey = mk(k12, k22);
+      NM = inverse(K);
+    } else {
+      vcount = 1;
+    }
+  }
+  ConFields f;
+  f.v[0] = make_float4(normal.x, normal.y, mat.x, mat.w);
+  f.v[1] = make_float4(mA, mB, iA, iB);
+  // point count, bit 8: the world warm-starts
+  f.v[2] = make_float4(as_float(ia), as_float(ib), as_float(vcount | (warm ? 256 : 0)), as_float(c));
+  f.v[3] = make_float4(rA0.x, rA0.y, rB0.x, rB0.y);
+  f.v[4] = make_float4(ni0, ti0, nm0, tm0);
+  f.v[5] = make_float4(rA1.x, rA1.y, rB1.x, rB1.y);
+  f.v[6] = make_float4(ni1, ti1, nm1, tm1);
+  f.v[7] = make_float4(bias0, bias1, K.ex.y, K.ey.x);
+  f.v[8] = make_float4(NM.ex.x, NM.ex.y, NM.ey.x, NM.ey.y);
+  f.v[9] = make_float4(K.ex.x, K.ex.y, K.ey.x, K.ey.y);
+  f.p[0] = make_float4(lp.x, lp.y, ln.x, ln.y);
+  f.p[1] = make_float4(lp0.x, lp0.y, lp1.x, lp1.y);
+  f.p[2] = make_float4(lcA.x, lcA.y, lcB.x, lcB.y);
+  f.p[3] = make_float4(mA, mB, iA, iB);
+  f.p[4] = make_float4(rA, rB, as_float(mtype), as_float(pcount));
+  return f;
+}
+
+__device__ __forceinline__ void contact_init(const Dev& d, int s) {
+  const int c = d.csorted[s];
+  const int2 pr = d.cpair[c];
+  const int4 ha = d.shdr[pr.x], hb = d.shdr[pr.y];
+  const int ia = ha.y, ib = hb.y;
+  const ConFields f = contact_fields(d, c, pr, ia, ib, ha.w, d.pos[ia], d.pos[ib], d.vel[ia], d.vel[ib]);
+  {  // this slot's place in each dynamic body's colour-ordered list (rank of
+     // its colour among the body's colours)
+    const int col = d.part_on ? -1 : d.ccol[c];
+    if (col >= 0 && col < kBodyTab) {
+      const unsigned long long below = (1ull << col) - 1ull;
+      if (d.btype[ia] == kDynamicBody) d.btab[(size_t)ia * kBodyTab + __popcll(d.bmask[ia] & below)] = 2 * s;
+      if (d.btype[ib] == kDynamicBody) d.btab[(size_t)ib * kBodyTab + __popcll(d.bmask[ib] & below)] = 2 * s + 1;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 10; ++k) d.vc[k][s] = f.v[k];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) d.pc[k][s] = f.p[k];
+}
+
 // (6 waves per SIMD: 80 registers, measured slightly faster than 5)
 __global__ void __launch_bounds__(kBlock, 6) k_contact_init(Dev d) {
   const int n = d.cnt[C_CONS];
-  B2G_FOR(s, 0, n) {
-    const int c = d.csorted[s];
-    const int2 pr = d.cpair[c];
-    const int4 ha = d.shdr[pr.x], hb = d.shdr[pr.y];
-    const int ia = ha.y, ib = hb.y;
-    const float4 pa = d.prop[ia], pb = d.prop[ib];
-    const float mA = pa.x, iA = pa.y, mB = pb.x, iB = pb.y;
-    const vec2 lcA = mk(pa.z, pa.w), lcB = mk(pb.z, pb.w);
-    const float4 m0 = d.cman[4 * (size_t)c + 0], m1 = d.cman[4 * (size_t)c + 1];
-    const float4 m2 = d.cman[4 * (size_t)c + 2], m3 = d.cman[4 * (size_t)c + 3];
-    const int mtype = as_int(m3.z) & 0xff;
-    const int count = (as_int(m3.z) >> 8) & 0xff;
-    const float4 mat = d.cmat[c];
-    const float rA = d.geo[9 * (size_t)pr.x].x, rB = d.geo[9 * (size_t)pr.y].x;
-    const int w = ha.w;
-    const float4 wp = d.wpar[w];
-    const bool warm = (d.wflag[w] & 1) != 0;
-    const float ratio = wp.w;
-
-    float ni0 = 0.0f, ti0 = 0.0f, ni1 = 0.0f, ti1 = 0.0f;
-    if (warm) {
-      ni0 = ratio * m0.z;
-      ti0 = ratio * m0.w;
-      ni1 = ratio * m1.z;
-      ti1 = ratio * m1.w;
-    }
-    const float4 posA = d.pos[ia], posB = d.pos[ib];
-    const float4 velA = d.vel[ia], velB = d.vel[ib];
-    const vec2 cA = mk(posA.x, posA.y), cB = mk(posB.x, posB.y);
-    const vec2 vA = mk(velA.x, velA.y), vB = mk(velB.x, velB.y);
-    const float wA = velA.z, wB = velB.z;
-    xform xfA, xfB;
-    xfA.q = rot_of(posA.z);
-    xfB.q = rot_of(posB.z);
-    xfA.p = cA - mul(xfA.q, lcA);
-    xfB.p = cB - mul(xfB.q, lcB);
-    // b2WorldManifold::Initialize (src/collision/b2_collision.cpp:26-90)
-    vec2 normal, wp0 = mk(0.0f, 0.0f), wp1 = mk(0.0f, 0.0f);
-    const vec2 ln = mk(m2.x, m2.y), lp = mk(m2.z, m2.w);
-    const vec2 lp0 = mk(m0.x, m0.y), lp1 = mk(m1.x, m1.y);
-    if (mtype == kManCircles) {
-      normal = mk(1.0f, 0.0f);
-      const vec2 pA = mul(xfA, lp);
-      const vec2 pB = mul(xfB, lp0);
-      if (dist_sq(pA, pB) > kEpsilon * kEpsilon) normal = normalize(pB - pA);
-      const vec2 qA = pA + rA * normal;
-      const vec2 qB = pB - rB * normal;
-      wp0 = 0.5f * (qA + qB);
-    } else if (mtype == kManFaceA) {
-      normal = mul(xfA.q, ln);
-      const vec2 plane = mul(xfA, lp);
-      {
-        const vec2 clip = mul(xfB, lp0);
-        const vec2 qA = clip + (rA - dot(clip - plane, normal)) * normal;
-        const vec2 qB = clip - rB * normal;
-        wp0 = 0.5f * (qA + qB);
-      }
-      if (count > 1) {
-        const vec2 clip = mul(xfB, lp1);
-        const vec2 qA = clip + (rA - dot(clip - plane, normal)) * normal;
-        const vec2 qB = clip - rB * normal;
-        wp1 = 0.5f * (qA + qB);
-      }
-    } else {
-      normal = mul(xfB.q, ln);
-      const vec2 plane = mul(xfB, lp);
-      {
-        const vec2 clip = mul(xfA, lp0);
-        const vec2 qB = clip + (rB - dot(clip - plane, normal)) * normal;
-        const vec2 qA = clip - rA * normal;
-        wp0 = 0.5f * (qA + qB);
-      }
-      if (count > 1) {
-        const vec2 clip = mul(xfA, lp1);
-        const vec2 qB = clip + (rB - dot(clip - plane, normal)) * normal;
-        const vec2 qA = clip - rA * normal;
-        wp1 = 0.5f * (qA + qB);
-      }
-      normal = -normal;
-    }
-    const vec2 tangent = cross(normal, 1.0f);
-    vec2 rA0 = wp0 - cA, rB0 = wp0 - cB, rA1 = wp1 - cA, rB1 = wp1 - cB;
-    float nm0, tm0, bias0 = 0.0f, nm1 = 0.0f, tm1 = 0.0f, bias1 = 0.0f;
-    {
-      const float rnA = cross(rA0, normal), rnB = cross(rB0, normal);
-      const float kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
-      nm0 = kn > 0.0f ? 1.0f / kn : 0.0f;
-      const float rtA = cross(rA0, tangent), rtB = cross(rB0, tangent);
-      const float kt = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
-      tm0 = kt > 0.0f ? 1.0f / kt : 0.0f;
-      const float vrel = dot(normal, vB + cross(wB, rB0) - (vA + cross(wA, rA0)));
-      if (vrel < -mat.z) bias0 = -mat.y * vrel;
-    }
-    if (count > 1) {
-      const float rnA = cross(rA1, normal), rnB = cross(rB1, normal);
-      const float kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
-      nm1 = kn > 0.0f ? 1.0f / kn : 0.0f;
-      const float rtA = cross(rA1, tangent), rtB = cross(rB1, tangent);
-      const float kt = mA + mB + iA * rtA * rtA + iB * rtB * rtB;
-      tm1 = kt > 0.0f ? 1.0f / kt : 0.0f;
-      const float vrel = dot(normal, vB + cross(wB, rB1) - (vA + cross(wA, rA1)));
-      if (vrel < -mat.z) bias1 = -mat.y * vrel;
-    }
-    int vcount = count, pcount = count;
-    if (d.sleep_on) {  // a sleeping island is not built (b2_world.cpp:535-539): no points to solve
-      const int isl = d.btype[ia] != kStaticBody ? d.parent[ia] : d.parent[ib];
-      if (d.isl_awake[isl]) d.isl_cons[isl] = 1;
-      else vcount = pcount = 0;
-    }
-    mat22 K = {mk(0.0f, 0.0f), mk(0.0f, 0.0f)}, NM = K;
-    if (count == 2 && vcount == 2) {  // block solver preparation (:236-256)
-      const float rn1A = cross(rA0, normal), rn1B = cross(rB0, normal);
-      const float rn2A = cross(rA1, normal), rn2B = cross(rB1, normal);
-      const float k11 = mA + mB + iA * rn1A * rn1A + iB * rn1B * rn1B;
-      const float k22 = mA + mB + iA * rn2A * rn2A + iB * rn2B * rn2B;
-      const float k12 = mA + mB + iA * rn1A * rn2A + iB * rn1B * rn2B;
-      const float kMaxCond = 1000.0f;
-      if (k11 * k11 < kMaxCond * (k11 * k22 - k12 * k12)) {
-        K.ex = mk(k11, k12);
-        K.ey = mk(k12, k22);
-        NM = inverse(K);
-      } else {
-        vcount = 1;
-      }
-    }
-    d.vc[0][s] = make_float4(normal.x, normal.y, mat.x, mat.w);
-    d.vc[1][s] = make_float4(mA, mB, iA, iB);
-    // point count, bit 8: the world warm-starts
-    d.vc[2][s] = make_float4(as_float(ia), as_float(ib), as_float(vcount | (warm ? 256 : 0)), as_float(c));
-    {  // this slot's place in each dynamic body's colour-ordered list (rank of
-       // its colour among the body's colours)
-      const int col = d.part_on ? -1 : d.ccol[c];
-      if (col >= 0 && col < kBodyTab) {
-        const unsigned long long below = (1ull << col) - 1ull;
-        if (d.btype[ia] == kDynamicBody) d.btab[(size_t)ia * kBodyTab + __popcll(d.bmask[ia] & below)] = 2 * s;
-        if (d.btype[ib] == kDynamicBody) d.btab[(size_t)ib * kBodyTab + __popcll(d.bmask[ib] & below)] = 2 * s + 1;
-      }
-    }
-    d.vc[3][s] = make_float4(rA0.x, rA0.y, rB0.x, rB0.y);
-    d.vc[4][s] = make_float4(ni0, ti0, nm0, tm0);
-    d.vc[5][s] = make_float4(rA1.x, rA1.y, rB1.x, rB1.y);
-    d.vc[6][s] = make_float4(ni1, ti1, nm1, tm1);
-    d.vc[7][s] = make_float4(bias0, bias1, K.ex.y, K.ey.x);
-    d.vc[8][s] = make_float4(NM.ex.x, NM.ex.y, NM.ey.x, NM.ey.y);
-    d.vc[9][s] = make_float4(K.ex.x, K.ex.y, K.ey.x, K.ey.y);
-    d.pc[0][s] = make_float4(lp.x, lp.y, ln.x, ln.y);
-    d.pc[1][s] = make_float4(lp0.x, lp0.y, lp1.x, lp1.y);
-    d.pc[2][s] = make_float4(lcA.x, lcA.y, lcB.x, lcB.y);
-    d.pc[3][s] = make_float4(mA, mB, iA, iB);
-    d.pc[4][s] = make_float4(rA, rB, as_float(mtype), as_float(pcount));
-  }
+  B2G_FOR(s, 0, n) contact_init(d, s);
 }
 
 __device__ __forceinline__ bool writes_body(const Dev& d, int b) { return d.btype[b] == kDynamicBody; }
@@ -1526,59 +1582,51 @@ __global__ void __launch_bounds__(kBlock) k_contact_velocity(Dev d, int colour, 
 // b2_island.cpp:621-647) goes to bits 16-23 of the manifold's packed word;
 // the narrowphase rewrites the word every step, so the bits name the points
 // the last step solved (0: not solved).
+__device__ __forceinline__ void store_contact_impulses(const Dev& d, int c, int count, float4 q0, float4 q1) {
+  float4* mp = d.cman + 4 * (size_t)c;
+  int* packed = reinterpret_cast<int*>(mp + 3) + 2;
+  *packed = (*packed & 0xffff) | (count << 16);
+  if (count == 0) return;  // not solved: the manifold keeps its impulses
+  *reinterpret_cast<float2*>(&mp[0].z) = make_float2(q0.x, q0.y);
+  if (count > 1) *reinterpret_cast<float2*>(&mp[1].z) = make_float2(q1.x, q1.y);
+}
 __device__ __forceinline__ void store_impulses(const Dev& d, int s) {
-  {
-    const float4 v2i = d.vc[2][s];
-    const int count = as_int(v2i.z) & 0xff, c = as_int(v2i.w);
-    const float4 q0 = d.vc[4][s];
-    float4* mp = d.cman + 4 * (size_t)c;
-    int* packed = reinterpret_cast<int*>(mp + 3) + 2;
-    *packed = (*packed & 0xffff) | (count << 16);
-    if (count == 0) return;  // not solved: the manifold keeps its impulses
-    float4 m0 = mp[0];
-    m0.z = q0.x;
-    m0.w = q0.y;
-    mp[0] = m0;
-    if (count > 1) {
-      const float4 q1 = d.vc[6][s];
-      float4 m1 = mp[1];
-      m1.z = q1.x;
-      m1.w = q1.y;
-      mp[1] = m1;
-    }
-  }
+  const float4 v2i = d.vc[2][s];
+  store_contact_impulses(d, as_int(v2i.w), as_int(v2i.z) & 0xff, d.vc[4][s], d.vc[6][s]);
 }
 
 // ===========================================================================
 // Position integration with the translation / rotation clamp
 // (src/dynamics/b2_island.cpp:341-385)
 // ===========================================================================
-__device__ __forceinline__ void integrate_position(const Dev& d, int b) {
-  {
-    const int w = d.bworld[b];
-    if (!world_active(d, w) || d.btype[b] == kStaticBody) return;
-    if (d.sleep_on && !d.bactive[b]) return;  // a sleeping island does not move
-    const float h = d.wpar[w].z;
-    const float4 v4 = d.vel[b];
-    vec2 v = mk(v4.x, v4.y);
-    float wv = v4.z;
-    const vec2 tr = h * v;
-    if (dot(tr, tr) > kMaxTranslationSq) {
-      const float ratio = kMaxTranslation / length(tr);
-      v = ratio * v;
-    }
-    const float rotation = h * wv;
-    if (rotation * rotation > kMaxRotationSq) {
-      const float ratio = kMaxRotation / absf(rotation);
-      wv *= ratio;
-    }
-    const float4 p = d.pos[b];
-    const vec2 c = mk(p.x, p.y) + h * v;
-    const float a = p.z + h * wv;
-    d.pos[b] = make_float4(c.x, c.y, a, 0.0f);
-    d.vel[b] = make_float4(v.x, v.y, wv, 0.0f);
-    if (d.flow_on) flow_start(d.fpos, b, c.x, c.y, a);
+// (the clamped velocity goes to v4)
+__device__ __forceinline__ float4 integrated_position(float h, float4 p, float4& v4) {
+  vec2 v = mk(v4.x, v4.y);
+  float wv = v4.z;
+  const vec2 tr = h * v;
+  if (dot(tr, tr) > kMaxTranslationSq) {
+    const float ratio = kMaxTranslation / length(tr);
+    v = ratio * v;
   }
+  const float rotation = h * wv;
+  if (rotation * rotation > kMaxRotationSq) {
+    const float ratio = kMaxRotation / absf(rotation);
+    wv *= ratio;
+  }
+  const vec2 c = mk(p.x, p.y) + h * v;
+  const float a = p.z + h * wv;
+  v4 = make_float4(v.x, v.y, wv, 0.0f);
+  return make_float4(c.x, c.y, a, 0.0f);
+}
+__device__ __forceinline__ void integrate_position(const Dev& d, int b) {
+  const int w = d.bworld[b];
+  if (!world_active(d, w) || d.btype[b] == kStaticBody) return;
+  if (d.sleep_on && !d.bactive[b]) return;  // a sleeping island does not move
+  float4 v = d.vel[b];
+  const float4 p = integrated_position(d.wpar[w].z, d.pos[b], v);
+  d.pos[b] = p;
+  d.vel[b] = v;
+  if (d.flow_on) flow_start(d.fpos, b, p.x, p.y, p.z);
 }
 
 // StoreImpulses for every solved contact and position integration for every
@@ -2319,25 +2367,22 @@ __global__ void __launch_bounds__(kBlock) k_clear_forces(Dev d) {
 // contacts of its shapes are contiguous in the key-sorted contact list and
 // keep their order in the compacted list. Also persists the colours and
 // advances the claim-round base (block 0).
-__global__ void __launch_bounds__(kBlock) k_world_colour_sort(Dev d, int rounds_run) {
+// The worlds of `order`, one per workgroup.
+__global__ void __launch_bounds__(kBlock) k_world_colour_sort(Dev d, int rounds_run, const int* order) {
   __shared__ int hist[kColourSlots];
   __shared__ int off[kColourSlots + 1];
   __shared__ int cur[kColourSlots];
   __shared__ int range[2];
-  const int w = d.worder[blockIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x == 0) d.cnt[C_ROUND] += rounds_run;
+  const int w = order[blockIdx.x];
   if (!world_active(d, w)) {  // no touching contact (the narrowphase left them all untouched): no colours
-    if (threadIdx.x == 0) {
-      if (blockIdx.x == 0) d.cnt[C_ROUND] += rounds_run;
-      d.wcolmax[w] = -1;
-    }
+    if (threadIdx.x == 0) d.wcolmax[w] = -1;
     return;  // the whole block
   }
   if (threadIdx.x == 0) {
-    if (blockIdx.x == 0) d.cnt[C_ROUND] += rounds_run;
-    const int nc = d.cnt[C_CONTACTS], total = d.cnt[C_CONS];
-    const int2 cr = world_contacts(d, w);
-    range[0] = cr.x < nc ? d.tpos[cr.x] : total;
-    range[1] = cr.y < nc ? d.tpos[cr.y] : total;
+    const int2 t = world_solved(d, w);
+    range[0] = t.x;
+    range[1] = t.y;
   }
   for (int c = threadIdx.x; c < kColourSlots; c += blockDim.x) {
     hist[c] = 0;

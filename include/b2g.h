@@ -283,7 +283,9 @@ int b2g_time_kernel(b2g_batch* batch, int32_t kernel);
 
 /* Solver layout and tuning. B2G_OPT_SOLVER: B2G_SOLVER_AUTO (default: one
  * workgroup per world when the batch has several joint-free worlds of at most
- * 8192 bodies laid out world after world; else colour-major sweeps),
+ * 8192 bodies laid out world after world, or a single one of at most 4096
+ * bodies that had at most 2048 contacts in its last step; else colour-major
+ * sweeps),
  * B2G_SOLVER_COLOURS (one launch
  * per colour over all worlds), B2G_SOLVER_WORLDS (one workgroup solves a
  * whole world, barriers between colours; needs that layout; the same results
@@ -292,10 +294,11 @@ int b2g_time_kernel(b2g_batch* batch, int32_t kernel);
  * workgroup with its bodies in LDS: three launches per iteration and no host
  * read per step; another valid constraint order, reported by
  * b2g_download_contact_colours as phase * 65536 + colour; on request only).
- * B2G_OPT_WORLD_BLOCK: threads per world workgroup, 0 = autotune: the first
- * per-world steps time 64..1024 threads, each with the world's bodies in
- * global memory and staged in LDS (when the largest world fits 63 KB), one
- * step per candidate, and keep the fastest.
+ * B2G_OPT_WORLD_BLOCK: threads per world workgroup, 0 = the engine's choice:
+ * eager steps solve worlds in workgroups by their contact counts, captured
+ * steps in workgroups of one fixed size. A size given here, or a B2G_OPT_WORLD_LDS
+ * of 0 or 1, holds for both. B2G_OPT_TUNED_WORLD_BLOCK is the size of a captured
+ * step's workgroups.
  * Read-only: B2G_OPT_TUNED_WORLD_BLOCK, B2G_OPT_LAST_SOLVER (1 colours,
  * 2 worlds, 3 cells), B2G_OPT_PER_WORLD_ELIGIBLE. No reference counterpart. */
 enum { B2G_SOLVER_AUTO = 0, B2G_SOLVER_COLOURS = 1, B2G_SOLVER_WORLDS = 2, B2G_SOLVER_CELLS = 3 };
@@ -305,7 +308,7 @@ enum {
   B2G_OPT_TUNED_WORLD_BLOCK = 3,
   B2G_OPT_LAST_SOLVER = 4,
   B2G_OPT_PER_WORLD_ELIGIBLE = 5,
-  B2G_OPT_WORLD_LDS = 6,        /* -1 autotune (default), 0 off, 1 stage each world's bodies in LDS */
+  B2G_OPT_WORLD_LDS = 6,        /* -1 the engine's choice (default), 0 off, 1 stage each world's bodies in LDS */
   B2G_OPT_TUNED_WORLD_LDS = 7,  /* read-only: whether the per-world solver stages bodies in LDS */
   /* 1 (default): a world that is not active in a step keeps its pairs and,
    * on the steps that refit the tree, its boxes and tree nodes, instead of
