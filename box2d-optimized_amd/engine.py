@@ -88,6 +88,7 @@ EXPORTS = [
     "b2g_time_kernel", "b2g_kernel_time", "b2a_scene_records", "b2a_batch_from_scenes", "b2s_run",
     "b2g_set_option", "b2g_get_option", "b2g_upload_contact_colours", "b2g_snapshot_save",
     "b2g_snapshot_load", "b2g_download_events", "b2g_query_aabbs", "b2g_raycast",
+    "b2g_query_aabbs_list", "b2g_raycast_list", "b2g_query_results",
     "b2g_set_counts", "b2g_download_solver_points", "b2a_world_destroy_body", "b2a_world_destroy_joint",
     "b2a_world_destroy_fixture", "b2a_world_set_filter", "b2a_world_body_count", "b2a_world_set_allow_sleep",
 ]
@@ -169,6 +170,9 @@ def lib():
         L.b2g_download_events.argtypes = [_P, _I, _P, _P]
         L.b2g_query_aabbs.argtypes = [_P, _I, _P, _P, _I, _P, _P]
         L.b2g_raycast.argtypes = [_P, _I, _P, _P, _I, _P, _P]
+        L.b2g_query_aabbs_list.argtypes = [_P, _I, _P, _P, _I, _P, _P]
+        L.b2g_raycast_list.argtypes = [_P, _I, _P, _P, _I, _P, _P]
+        L.b2g_query_results.argtypes = [_P, _P]
         L.b2g_snapshot_load.argtypes = [_P, ctypes.c_char_p]
         L.b2g_get_option.argtypes = [_P, _I, _P]
         L.b2g_set_counts.argtypes = [_P, _I, _I, _I]
@@ -341,25 +345,23 @@ class Batch:
         """Shapes overlapping each AABB: list of int arrays (b2g_query_aabbs)."""
         w = np.ascontiguousarray(worlds, dtype=np.int32)
         a = np.ascontiguousarray(aabbs, dtype=np.float32).reshape(len(w), 4)
-        while True:
-            out = np.zeros((len(w), capacity), np.int32)
-            cnt = np.zeros(len(w), np.int32)
-            check(self.L.b2g_query_aabbs(self.h, len(w), _ptr(w), _ptr(a), capacity, _ptr(out), _ptr(cnt)))
-            if len(cnt) == 0 or cnt.max() <= capacity:
-                return [out[i, :cnt[i]].copy() for i in range(len(w))]
-            capacity = int(cnt.max())
+        return self._query(self.L.b2g_query_aabbs_list, w, a, capacity, np.int32)
 
     def raycast(self, worlds, segments, capacity=64):
         """All hits of each segment (p1, p2): list of RAY_HIT_DTYPE arrays (b2g_raycast)."""
         w = np.ascontiguousarray(worlds, dtype=np.int32)
         sg = np.ascontiguousarray(segments, dtype=np.float32).reshape(len(w), 4)
-        while True:
-            out = np.zeros((len(w), capacity), RAY_HIT_DTYPE)
-            cnt = np.zeros(len(w), np.int32)
-            check(self.L.b2g_raycast(self.h, len(w), _ptr(w), _ptr(sg), capacity, _ptr(out), _ptr(cnt)))
-            if len(cnt) == 0 or cnt.max() <= capacity:
-                return [out[i, :cnt[i]].copy() for i in range(len(w))]
-            capacity = int(cnt.max())
+        return self._query(self.L.b2g_raycast_list, w, sg, capacity, RAY_HIT_DTYPE)
+
+    def _query(self, run, worlds, boxes, capacity, dtype):
+        cnt = np.zeros(len(worlds), np.int32)
+        total = ctypes.c_int64(0)
+        check(run(self.h, len(worlds), _ptr(worlds), _ptr(boxes), capacity, _ptr(cnt), ctypes.byref(total)))
+        out = np.empty(total.value, dtype)
+        if total.value:
+            check(self.L.b2g_query_results(self.h, _ptr(out)))
+        end = np.cumsum(cnt, dtype=np.int64).tolist()
+        return [out[e - n:e].copy() for e, n in zip(end, cnt.tolist())]
 
     def events(self):
         """Contact events of the last step taken with STEP_EVENTS."""

@@ -397,6 +397,16 @@ int b2g_query_aabbs(b2g_batch* batch, int32_t n, const int32_t* worlds, const fl
                     int32_t* out_shapes, int32_t* out_counts);
 int b2g_raycast(b2g_batch* batch, int32_t n, const int32_t* worlds, const float* segments, int32_t capacity,
                 b2g_ray_hit* out_hits, int32_t* out_counts);
+/* The same queries with all their results, one query after the other: the
+ * first call runs them (`capacity`: the results of one query that its first
+ * pass has room for; any number is found) and gives each query's count and
+ * the total, b2g_query_results then writes that many records (int32_t shapes
+ * or b2g_ray_hit) to `out`, once, before the batch's next query. */
+int b2g_query_aabbs_list(b2g_batch* batch, int32_t n, const int32_t* worlds, const float* aabbs, int32_t capacity,
+                         int32_t* out_counts, int64_t* total);
+int b2g_raycast_list(b2g_batch* batch, int32_t n, const int32_t* worlds, const float* segments, int32_t capacity,
+                     int32_t* out_counts, int64_t* total);
+int b2g_query_results(b2g_batch* batch, void* out);
 
 /* Binary snapshot of a batch: capacity, world params, bodies, shapes,
  * joints with their impulses, contacts with manifolds, impulses and colours.
