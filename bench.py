@@ -177,8 +177,8 @@ def batched_section(pkg, worlds: int, warmup: int, steps: int, sample_every: int
     el = timed(batch, mode)
     counts = batch.counts()
     solver = {"path": "per-world workgroups" if batch.get_option(eng.OPT_LAST_SOLVER) == 2 else "colour sweeps",
-              "tuned_workgroup": batch.get_option(eng.OPT_TUNED_WORLD_BLOCK),
-              "tuned_lds_bodies": bool(batch.get_option(eng.OPT_TUNED_WORLD_LDS))}
+              "captured_workgroup": batch.get_option(eng.OPT_TUNED_WORLD_BLOCK),
+              "captured_lds_bodies": bool(batch.get_option(eng.OPT_TUNED_WORLD_LDS))}
     batch.close()
     # the same steps (a second batch of the same worlds, advanced alike) in
     # the other launch mode: replays of the captured step graph, or eager
