@@ -23,6 +23,7 @@
 #include "b2g_partition.h"
 #include "b2g_flow.h"
 #include "b2g_worlds.h"
+#include "b2g_joints.h"
 
 using namespace b2g;
 
@@ -327,7 +328,7 @@ int b2g_batch::alloc() {
   A(d.joints, NJ); A(d.jsol, NJ); A(d.jorder, NJ); A(d.jisland, NJ); A(d.wj_off, NW + 1); A(d.wj_list, NJ);
   A(d.bj_off, NB + 1); A(d.bj_other, 2 * NJ);
   A(d.flow_ctl, kFlowCtl);
-  A(d.jcol_off, kMaxColours + 1); A(d.jrank, NJ); A(d.bjdeg, NB);
+  A(d.jcol_off, kMaxColours + 1); A(d.jplace, NJ); A(d.bjdeg, NB);
   A(d.ckey, NC); A(d.cpair, NC); A(d.cman, 4 * (size_t)NC); A(d.cmat, NC); A(d.ccol, NC);
   A(d.nkey, NC); A(d.npair, NC); A(d.nman, 4 * (size_t)NC); A(d.nmat, NC); A(d.ncol, NC);
   A(d.touch, NC); A(d.tpos, NC); A(d.clist, NC); A(d.cbody, NC); A(d.ccolour, NC); A(d.csorted, NC);
@@ -450,7 +451,7 @@ void b2g_batch::release() {
                   d.gltab, d.gloff, d.sfast, d.sparse, d.pslots, d.heavy, d.pcount, d.pfound, d.sinv, d.poff, d.poff_prev, d.scan_tiles,
                   d.cnt,
                   // the flow solver
-                  d.fvel, d.fpos, d.flow_ctl, d.jcol_off, d.jrank, d.bjdeg,
+                  d.fvel, d.fpos, d.flow_ctl, d.jcol_off, d.jplace, d.bjdeg,
                   // sleep
                   d.bsflag, d.bstime, d.bwake, d.bactive, d.bncontact, d.bjointed, d.isl_awake, d.isl_min, d.isl_cons,
                   // the cells solver
@@ -799,44 +800,19 @@ int b2g_batch::finish_pair_list(bool use_given_aabbs) {
 // upload), plus the CSR of joint partners that must not collide.
 int b2g_batch::rebuild_joint_tables() {
   const int nj = d.nj, nb = d.nb;
-  std::vector<unsigned long long> used(std::max(nb, 1), 0ull);
-  std::vector<int> col(nj, 0);
-  int ncol = 0;
-  for (int q = 0; q < nj; ++q) {
-    const b2g_revolute& j = h_joints[q];
-    unsigned long long m = 0;
-    const bool da = h_btype[j.body_a] == B2G_DYNAMIC, db = h_btype[j.body_b] == B2G_DYNAMIC;
-    if (da) m |= used[j.body_a];
-    if (db) m |= used[j.body_b];
-    int c = 0;
-    while (c < 64 && (m >> c) & 1ull) ++c;
-    if (c >= 64) return fail(B2G_ERR_CAPACITY, "joint graph needs more than 64 colours");
-    col[q] = c;
-    if (da) used[j.body_a] |= 1ull << c;
-    if (db) used[j.body_b] |= 1ull << c;
-    ncol = std::max(ncol, c + 1);
-  }
-  std::vector<int> order(nj);
-  h_jcol_off.assign(ncol + 1, 0);
-  for (int q = 0; q < nj; ++q) h_jcol_off[col[q] + 1]++;
-  for (int c = 0; c < ncol; ++c) h_jcol_off[c + 1] += h_jcol_off[c];
-  std::vector<int> cur(h_jcol_off.begin(), h_jcol_off.end());
-  for (int q = 0; q < nj; ++q) order[cur[col[q]]++] = q;
-  {  // each joint's place in its bodies' update sequences (joints of a body differ in colour)
-    std::vector<int> deg(std::max(nb, 1), 0), offs(kMaxColours + 1, 0);
-    std::vector<int2> rank(std::max(nj, 1));
-    for (int k = 0; k < nj; ++k) {
-      const b2g_revolute& j = h_joints[order[k]];
-      rank[k].x = deg[j.body_a] | col[order[k]] << 8;
-      rank[k].y = deg[j.body_b];
-      ++deg[j.body_a];
-      if (j.body_b != j.body_a) ++deg[j.body_b];
-    }
-    for (int c = 0; c <= ncol; ++c) offs[c] = h_jcol_off[c];
-    d.njcol = ncol;
-    if (nb) HIP_TRY(hipMemcpy(d.bjdeg, deg.data(), nb * sizeof(int), hipMemcpyHostToDevice));
-    if (nj) HIP_TRY(hipMemcpy(d.jrank, rank.data(), nj * sizeof(int2), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d.jcol_off, offs.data(), offs.size() * sizeof(int), hipMemcpyHostToDevice));
+  JointTables t;
+  if (!joint_tables(nj, nb, [&](int q) -> const b2g_revolute& { return h_joints[q]; },
+                    [&](int b) { return h_btype[b] == B2G_DYNAMIC; }, &t))
+    return fail(B2G_ERR_CAPACITY, "joint graph needs more than 64 colours");
+  h_jcol_off = t.offsets;
+  {
+    static_assert(kMaxJointColours <= kMaxColours, "d.jcol_off holds every joint colour's offset");
+    std::vector<int2> place(std::max(nj, 1));
+    for (int k = 0; k < nj; ++k) place[k] = make_int2(pack_joint_ranks(t.places[k]), t.places[k].colour);
+    d.njcol = (int)t.offsets.size() - 1;
+    if (nb) HIP_TRY(hipMemcpy(d.bjdeg, t.degree.data(), nb * sizeof(int), hipMemcpyHostToDevice));
+    if (nj) HIP_TRY(hipMemcpy(d.jplace, place.data(), nj * sizeof(int2), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(d.jcol_off, t.offsets.data(), t.offsets.size() * sizeof(int), hipMemcpyHostToDevice));
   }
   // CSR of non-colliding joint partners
   std::vector<int> off(nb + 1, 0), other;
@@ -858,7 +834,7 @@ int b2g_batch::rebuild_joint_tables() {
     for (int q = 0; q < nj; ++q) jointed[h_joints[q].body_a] = jointed[h_joints[q].body_b] = 1;
     if (nb) HIP_TRY(hipMemcpy(d.bjointed, jointed.data(), nb * sizeof(int), hipMemcpyHostToDevice));
   }
-  if (nj) HIP_TRY(hipMemcpy(d.jorder, order.data(), nj * sizeof(int), hipMemcpyHostToDevice));
+  if (nj) HIP_TRY(hipMemcpy(d.jorder, t.order.data(), nj * sizeof(int), hipMemcpyHostToDevice));
   {  // joints grouped by world (of body A), for the per-world island pass
     const int nw = d.nw;
     std::vector<int> woff(nw + 1, 0), wlist(std::max(nj, 1));
@@ -2116,6 +2092,8 @@ int b2g_upload_bodies(b2g_batch* b, int32_t first, int32_t count, const b2g_body
     type[i] = s.type;
     world[i] = s.world;
     if (b->h_bworld[first + i] != s.world) b->layout_dirty = true;
+    // joint colours and places go by which bodies are dynamic
+    if (!b->h_joints.empty() && b->h_btype[first + i] != s.type) b->joints_dirty = true;
     b->h_btype[first + i] = s.type;
     b->h_bworld[first + i] = s.world;
   }

@@ -273,9 +273,9 @@ __device__ __forceinline__ void flow_velocity_joint(const Dev& d, int q, bool va
   if (valid) {
     ji = d.jorder[q];
     j = d.joints[ji];
-    rank = d.jrank[q];
-    key = rank.x >> 8;
-    rank.x &= 0xff;
+    const int2 place = d.jplace[q];
+    key = place.y;
+    rank = make_int2(place.x & 0xff, place.x >> 8);
     const float4 wp = d.wpar[j.world];
     h = wp.z;
     ratio = wp.w;
@@ -502,9 +502,9 @@ __device__ __forceinline__ void flow_position_joint(const Dev& d, int q, bool va
   if (valid) {
     j = d.joints[d.jorder[q]];
     js = d.jsol[q];
-    rank = d.jrank[q];
-    key = rank.x >> 8;
-    rank.x &= 0xff;
+    const int2 place = d.jplace[q];
+    key = place.y;
+    rank = make_int2(place.x & 0xff, place.x >> 8);
     const float4 ca = d.pos[j.a], cb = d.pos[j.b];
     sa[0] = ca.x; sa[1] = ca.y; sa[2] = ca.z;
     sb[0] = cb.x; sb[1] = cb.y; sb[2] = cb.z;

@@ -242,9 +242,8 @@ struct Dev {
   int* flow_ctl;      // kFlowCtl words: arrival counts and go words of the step's flow launches
   int* jcol_off;      // offsets of the joint colours (kMaxColours + 1)
   int njcol;          // joint colours
-  int2* jrank;        // per colour-ordered joint: its place among each body's joints, in colour order (x: its
-                      // colour above bit 8)
-  int* bjdeg;         // per body: joints attached to it
+  int2* jplace;       // per colour-ordered joint: its rank among each body's joints (x, pack_joint_ranks), its colour (y)
+  int* bjdeg;         // per dynamic body: joints attached to it
   int* part_xcol;     // per cross-group constraint: its colour while colouring
   int2* sloc;         // per slot: LDS slots of its two bodies in its cell (-1: global memory)
 };

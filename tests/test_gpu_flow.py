@@ -33,6 +33,22 @@ def _motors(n=70):
     return s
 
 
+def _pendulums(single, double):
+    """Pendulums apart from each other, every anchor on the static body 0, the last `double` with a second link."""
+    s = S.Scene(name="pendulums", gravity=(0.0, -10.0))
+    s.add_body(S.STATIC, 0.0, 0.0)
+    at = [(4.0 * (i % 250), 5.0 * (i // 250)) for i in range(single + double)]
+    for x, y in at:
+        s.add_box(s.add_body(S.DYNAMIC, x + 0.5, y), 0.4, 0.1)
+    for x, y in at[single:]:
+        s.add_box(s.add_body(S.DYNAMIC, x + 1.5, y), 0.4, 0.1)
+    for i, (x, y) in enumerate(at):
+        s.add_revolute(0, 1 + i, (x, y))
+    for i, (x, y) in enumerate(at[single:]):
+        s.add_revolute(1 + single + i, 1 + single + double + i, (x + 1.0, y))
+    return s
+
+
 def _sleepers():
     import make_golden
     return make_golden.sleep_scene()
@@ -51,6 +67,9 @@ CASES = {
     "gas_chains": ([lambda: S.gas_and_chains(4000, 16, 30, seed=0x5C3, half=80.0)], 30, 8, 3, True, False),
     "worlds_with_joints": ([lambda: S.gas_and_chains(300, 4, 9, seed=1, half=25.0), _motors,
                             lambda: S.random_pile(200, seed=2, half_w=9.0, height=30.0)], 50, 8, 3, True, False),
+    # more joints on one static body than a byte counts; the first second link shares a wavefront with its anchor
+    "pendulums_two_to_a_wave": ([lambda: _pendulums(1200, 1)], 40, 8, 3, True, False),
+    "pendulums_64_to_a_wave": ([lambda: _pendulums(64990, 10)], 10, 8, 3, True, False),
     "sleep": ([_sleepers], 200, 8, 3, True, True),
     "sleep_joints": ([lambda: S.gas_and_chains(300, 6, 12, seed=7, half=40.0)], 120, 8, 3, True, True),
 }
@@ -89,3 +108,24 @@ def test_gpu_sweeps_past_the_resident_limit_use_a_launch_per_colour(engine):
     b = engine.Batch.from_scenes([sc]).advance(2)
     assert b.get_option(engine.OPT_LAST_SWEEPS) == 1
     b.close()
+
+
+def test_gpu_a_jointed_body_that_turns_dynamic_gets_a_place_in_its_joints_order(engine):
+    """Which joints of a body must differ in colour, and its joints' ranks, go by the body's type."""
+    sc = _motors()
+    lift = [i for i, t in enumerate(sc.body_type) if t == S.KINEMATIC][0]
+    batches = []
+    for mode in (1, 0):
+        b = engine.Batch.from_scenes([sc])
+        b.set_option(engine.OPT_SOLVER, engine.SOLVER_COLOURS)
+        b.set_option(engine.OPT_SWEEPS, mode)
+        b.advance(10)
+        rec = b.bodies()
+        rec["type"][lift], rec["mass"][lift], rec["inv_mass"][lift], rec["inv_i"][lift] = S.DYNAMIC, 2.0, 0.5, 0.3
+        b.upload_bodies(0, rec)
+        b.advance(30)
+        batches.append(b)
+    ref, b = batches
+    assert b.get_option(engine.OPT_LAST_SWEEPS) == 2
+    assert np.array_equal(ref.bodies().view(np.uint8), b.bodies().view(np.uint8))
+    assert np.array_equal(ref.joints(sc.joint_count).view(np.uint8), b.joints(sc.joint_count).view(np.uint8))
