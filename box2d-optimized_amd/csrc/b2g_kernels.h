@@ -2364,15 +2364,16 @@ __global__ void __launch_bounds__(kBlock) k_clear_forces(Dev d) {
 // ===========================================================================
 // Slots of world w's constraints (world-major, colour-minor): the touching
 // contacts of its shapes are contiguous in the key-sorted contact list and
-// keep their order in the compacted list. Also persists the colours and
-// advances the claim-round base (block 0).
+// keep their order in the compacted list. Also persists the colours and, with
+// `rounds_run`, advances the claim-round base (block 0): one launch of a step
+// does, so a launch beside another that does has 0 and leaves it alone.
 // The worlds of `order`, one per workgroup.
 __global__ void __launch_bounds__(kBlock) k_world_colour_sort(Dev d, int rounds_run, const int* order) {
   __shared__ int hist[kColourSlots];
   __shared__ int off[kColourSlots + 1];
   __shared__ int cur[kColourSlots];
   __shared__ int range[2];
-  if (blockIdx.x == 0 && threadIdx.x == 0) d.cnt[C_ROUND] += rounds_run;
+  if (rounds_run && blockIdx.x == 0 && threadIdx.x == 0) d.cnt[C_ROUND] += rounds_run;
   const int w = order[blockIdx.x];
   if (!world_active(d, w)) {  // no touching contact (the narrowphase left them all untouched): no colours
     if (threadIdx.x == 0) d.wcolmax[w] = -1;

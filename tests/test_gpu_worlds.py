@@ -91,3 +91,19 @@ def test_gpu_worlds_by_class_with_idle_worlds(engine):
             x.set_world_params(0, [engine.WorldParams(g, dt, 1.0, 1, int(on[w])) for w, g in enumerate(x.gravity)])
             x.step(8, 3, 0)
         _same(a, b, k)
+
+
+def test_gpu_worlds_past_the_largest_class_keep_the_claim_rounds(engine):
+    """One launch of a step moves the claim-round base on, also where the largest worlds' launches run beside
+    the classes': with a base that lags, old claims win and colours change. Colours of every step."""
+    big = S.random_pile(2600, seed=8, half_w=26.0, height=60.0)
+    a, b = _pair(engine, [big] + [S.batch_world(i, 20 + 25 * i) for i in range(12)])
+    a.advance(100)
+    b.advance(100)
+    for k in range(60):
+        a.advance(1)
+        b.advance(1)
+        n = len(a.contacts())
+        assert np.array_equal(a.contact_colours(n), b.contact_colours(n)), k
+    _same(a, b, "end")
+    assert a.counts().touching > 2048  # (the large world is past the largest class by far)
