@@ -1055,10 +1055,10 @@ void b2g_batch::enqueue_colour_groups() {
 // The coming step's sweeps may be ordered by data: the bodies' flow states
 // exist from the first such step on (a batch that only ever takes the
 // per-world solver does without their 256 bytes per body). Without room for
-// them the step launches its colours one by one.
+// them, or past the launches' reach, the step launches its colours one by one.
 void b2g_batch::use_flow() {
   d.flow_on = 0;
-  if (sweeps == 1) return;
+  if (sweeps == 1 || !flow_reaches(cap.bodies)) return;
   const size_t bytes = (size_t)kFlowStride * std::max(cap.bodies, 1);
   for (unsigned long long** p : {&d.fvel, &d.fpos})
     if (!*p && hipMalloc((void**)p, bytes) != hipSuccess) {

@@ -87,7 +87,8 @@ __device__ __forceinline__ bool flow_enter(int* ctl, long long wait, bool* sole)
 }
 
 // The bodies' states (Dev::fvel or Dev::fpos) behind a buffer descriptor: its
-// loads take a cache policy, and one that goes past the XCD's own L2.
+// loads take a cache policy, and one that goes past the XCD's own L2. (Sizes
+// and offsets are 32-bit: flow_reaches bounds the bodies.)
 typedef unsigned flow_u4 __attribute__((ext_vector_type(4)));
 struct FlowStates {
   __amdgpu_buffer_rsrc_t rsrc;

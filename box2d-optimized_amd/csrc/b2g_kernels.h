@@ -14,6 +14,7 @@
 #pragma once
 
 #include "b2g_collide.h"
+#include "b2g_flow_rule.h"
 #include "b2g_prims.h"
 #include <climits>
 
@@ -84,10 +85,6 @@ __device__ __host__ __forceinline__ constexpr int class_slots(int c) {
 __device__ __host__ __forceinline__ constexpr int class_bodies(int c) {
   return c == kPairClass ? kGroupBodies : kGroupBodies / 2 / class_worlds(c);
 }
-// bytes from one body's flow state to the next: a cache line each (16 bytes,
-// eight bodies to a line: 322 us per velocity phase of a settled pile of
-// 20,000 against 242)
-constexpr int kFlowStride = 128;
 struct Dev {
   int nb, ns, nj, nw;
   // bodies
