@@ -1277,7 +1277,7 @@ int b2g_batch::status_error() const {
     return fail(B2G_ERR_CAPACITY, "contact capacity exceeded (" + std::to_string(pinned[C_PAIRS]) + " pairs)");
   if (s & S_STACK_OVERFLOW) return fail(B2G_ERR_CAPACITY, "BVH traversal stack overflow");
   if (s & S_TREE_CORRUPT) return fail(B2G_ERR_INVALID, "BVH inconsistent (sort/build)");
-  if (s & S_FLOW_STALL) return fail(B2G_ERR_INVALID, "a constraint waited two seconds for its bodies");
+  if (s & S_FLOW_STALL) return fail(B2G_ERR_INVALID, "a constraint's bodies never came to its turn");
   return B2G_OK;
 }
 

@@ -41,7 +41,13 @@ constexpr int kFlowMaxPosIters = kFlowCtl - kFlowBar;
 constexpr int kFlowSpread = 1024;
 enum FlowGo : int { kFlowWait = 0, kFlowRun = 1, kFlowWithdrawn = 2 };
 constexpr long long kFlowEnterTicks = 100000;       // 1 ms of the 100 MHz clock
-constexpr long long kFlowStallTicks = 200000000ll;  // 2 s of the 100 MHz clock
+// Polls of a wait in which nothing comes, one memory round trip (0.5 us) each,
+// after which a count is taken to be broken: counted from the last progress,
+// and in polls rather than by the clock, so that neither a long phase nor a
+// preempted queue runs into it.
+constexpr int kFlowStallPolls = 1 << 22;          // a constraint: two seconds
+constexpr int kFlowMeetPolls = 2 * kFlowStallPolls;  // a meeting: past any constraint's
+constexpr int kFlowStalled = 1 << 20;  // added to a meeting's count: a constraint has stalled, all leave
 
 __device__ __forceinline__ int flow_load(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -139,16 +145,15 @@ __device__ __forceinline__ int flow_least(bool active, int key) {
 // us of one wave's issue slots, then serves one or two of them.) `step`
 // solves and posts, moves the lane on to its next wants and key, and says
 // whether it has more to do. The update of the least key of all waves never
-// waits, so some wave always goes on. A guard against a broken count ends the
-// loop after two seconds.
+// waits, so some wave always goes on. False: the wave stalled (a broken count)
+// and gave up.
 template <class Step>
-__device__ __forceinline__ void flow_run(const Dev& d, const FlowStates& f, bool active, int& key, FlowBody& A,
+__device__ __forceinline__ bool flow_run(const Dev& d, const FlowStates& f, bool active, int& key, FlowBody& A,
                                          FlowBody& B, float* sa, float* sb, Step step) {
   bool wa = A.waits(), wb = B.waits();
-  const long long t0 = wall_clock64();
   int least = flow_least(active, key);
   const bool mixed = __ballot(active && key != least) != 0;  // most waves hold one colour
-  for (unsigned pass = 1; least != INT_MAX; ++pass) {
+  for (int idle = 0; least != INT_MAX;) {
     const bool mine = active && (!mixed || key == least);
     if (__ballot(mine && (wa || wb)) != 0) {
       if (mine && (wa || wb)) {
@@ -158,7 +163,12 @@ __device__ __forceinline__ void flow_run(const Dev& d, const FlowStates& f, bool
         if (wa && flow_land(a, A, sa)) wa = false;
         if (wb && flow_land(b, B, sb)) wb = false;
       }
+      if (++idle > kFlowStallPolls) {
+        if (active) atomicOr(&d.cnt[C_STATUS], S_FLOW_STALL);
+        return false;
+      }
     } else {
+      idle = 0;
       if (mine) {
         active = step();
         wa = A.waits();
@@ -169,11 +179,8 @@ __device__ __forceinline__ void flow_run(const Dev& d, const FlowStates& f, bool
       else if (__ballot(active) == 0)
         least = INT_MAX;
     }
-    if ((pass & 1023u) == 0 && wall_clock64() - t0 > kFlowStallTicks) {
-      if (active) atomicOr(&d.cnt[C_STATUS], S_FLOW_STALL);
-      break;
-    }
   }
+  return true;
 }
 
 // the lane's constraint: `per` to a wave, in its first lanes (-1: none)
@@ -388,21 +395,27 @@ __global__ void __launch_bounds__(kFlowThreads, 4) k_flow_velocity(Dev d, int co
 // ---------------------------------------------------------------------------
 // All workgroups of the launch (they are resident): each marks its islands
 // with agent-scope stores, waits for them to be done, and counts itself in.
-__device__ __forceinline__ void flow_meet(const Dev& d, int* count, int blocks) {
+// `ok`: this wave did not stall; false where any of the launch did, in every
+// workgroup alike.
+__device__ __forceinline__ bool flow_meet(const Dev& d, int* count, int blocks, bool ok) {
+  __shared__ int s_met;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have reached the memory side
-  __syncthreads();
+  const bool stalled = __syncthreads_or(!ok) != 0;
   if (threadIdx.x == 0) {
-    const long long t0 = wall_clock64();
-    __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (unsigned turn = 1; flow_load(count) < blocks; ++turn) {
-      if ((turn & 255u) == 0 && wall_clock64() - t0 > kFlowStallTicks) {
+    __hip_atomic_fetch_add(count, stalled ? kFlowStalled : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int met = flow_load(count);
+    for (int polls = 0; met < blocks; met = flow_load(count)) {
+      if (++polls > kFlowMeetPolls) {
         atomicOr(&d.cnt[C_STATUS], S_FLOW_STALL);
+        met = kFlowStalled;
         break;
       }
     }
+    s_met = met;
   }
   __syncthreads();
+  return s_met < kFlowStalled;
 }
 
 // Whether the island is through before iteration `it` (island_done, from the
@@ -463,7 +476,7 @@ __device__ __forceinline__ void flow_position_contact(const Dev& d, int s, bool 
     A.want = (unsigned)(it * (nA + jA) + rA) & 0xffffu;
     B.want = (unsigned)(it * (nB + jB) + rB) & 0xffffu;
     bool bad = false;
-    flow_run(d, f, valid, key, A, B, sa, sb, [&]() {
+    const bool through = flow_run(d, f, valid, key, A, B, sa, sb, [&]() {
       PosPair u{mk(sa[0], sa[1]), mk(sb[0], sb[1]), sa[2], sb[2]};
       const float m = contact_position_core(r.p[0], r.p[1], r.p[2], r.p[3], r.p[4], u);
       bad = separation_bad(m);
@@ -484,7 +497,7 @@ __device__ __forceinline__ void flow_position_contact(const Dev& d, int s, bool 
     bad = bad && __hip_atomic_load(d.sepbad + island_slot(d, r.isl, it), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT) == 0u;
     mark_island_sep(d, it, valid ? r.isl : 0, bad, -1.0f);
-    if (it + 1 < pi) flow_meet(d, bar + it, (int)gridDim.x);
+    if (it + 1 < pi && !flow_meet(d, bar + it, (int)gridDim.x, through)) return;
   }
 }
 
@@ -525,7 +538,7 @@ __device__ __forceinline__ void flow_position_joint(const Dev& d, int q, bool va
     if (valid && flow_island_done(d, isl, it, pi)) valid = false;
     A.want = (unsigned)(it * (nA + jA) + nA + rank.x) & 0xffffu;
     B.want = (unsigned)(it * (nB + jB) + nB + rank.y) & 0xffffu;
-    flow_run(d, f, valid, key, A, B, sa, sb, [&]() {
+    const bool through = flow_run(d, f, valid, key, A, B, sa, sb, [&]() {
       PosPair u{mk(sa[0], sa[1]), mk(sb[0], sb[1]), sa[2], sb[2]};
       const bool ok = joint_position_core(j, js, u);
       if (A.body >= 0) {
@@ -541,7 +554,7 @@ __device__ __forceinline__ void flow_position_joint(const Dev& d, int q, bool va
       if (!ok) __hip_atomic_store(d.jok + island_slot(d, isl, it), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
     });
-    if (it + 1 < pi) flow_meet(d, bar + it, (int)gridDim.x);
+    if (it + 1 < pi && !flow_meet(d, bar + it, (int)gridDim.x, through)) return;
   }
 }
 

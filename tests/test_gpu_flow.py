@@ -129,3 +129,26 @@ def test_gpu_a_jointed_body_that_turns_dynamic_gets_a_place_in_its_joints_order(
     assert b.get_option(engine.OPT_LAST_SWEEPS) == 2
     assert np.array_equal(ref.bodies().view(np.uint8), b.bodies().view(np.uint8))
     assert np.array_equal(ref.joints(sc.joint_count).view(np.uint8), b.joints(sc.joint_count).view(np.uint8))
+
+
+def test_gpu_a_phase_of_many_seconds_is_no_stall(engine):
+    """Twenty spokes on one hub, their sweeps a chain of twenty updates an iteration, for so many iterations that
+    the launch takes seconds and the bodies' update counts wrap their 16 bits many times."""
+    s = S.Scene(name="star", gravity=(0.0, -10.0))
+    s.add_body(S.STATIC, 0.0, 0.0)
+    hub = s.add_body(S.DYNAMIC, 0.0, 0.0)
+    s.add_circle(hub, 0.3)
+    for i in range(20):
+        x, y = np.cos(0.31 * i), np.sin(0.31 * i)
+        arm = s.add_body(S.DYNAMIC, 2.0 * x, 2.0 * y)
+        s.add_box(arm, 0.1, 0.05)
+        s.add_revolute(hub, arm, (x, y))
+    batches = []
+    for mode in (0, 2):
+        b = engine.Batch.from_scenes([s])
+        b.set_option(engine.OPT_SWEEPS, mode)
+        b.advance(1, vi=120000, pi=20)
+        assert b.get_option(engine.OPT_LAST_SWEEPS) == 2
+        batches.append(b)
+    assert np.array_equal(batches[0].bodies().view(np.uint8), batches[1].bodies().view(np.uint8))
+    assert np.isfinite(batches[0].bodies()["v"]).all()
