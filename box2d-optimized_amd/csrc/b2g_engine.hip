@@ -212,6 +212,8 @@ struct b2g_batch {
   bool keep_idle = true;     // B2G_OPT_KEEP_IDLE
   int pair_search = 0;       // B2G_OPT_PAIR_SEARCH
   int sweeps = 0;            // B2G_OPT_SWEEPS
+  int flow_max_blocks = 0;   // workgroups of a flow launch that the device keeps resident
+  FlowRest flow_rest;
   int last_sweeps = 0;       // 1 a launch per colour, 2 ordered by data (k_flow_velocity, k_flow_position)
   int last_pair_search = 0;  // 1 LBVH, 2 grid
   int world_static_max = 0;  // most static shapes in one world
@@ -379,6 +381,7 @@ int b2g_batch::alloc() {
   d.ecap = NC;
   if ((rc = stage_room(std::min(kStageBytes, sizeof(b2g_body) * (size_t)NB))) != B2G_OK) return rc;
   HIP_TRY(hipHostMalloc((void**)&pinned, 256 * sizeof(int), hipHostMallocDefault));
+  std::memset(pinned, 0, 256 * sizeof(int));
   HIP_TRY(hipHostMalloc((void**)&stage_wpar, (size_t)NW * sizeof(float4), hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&stage_wflag, (size_t)NW * sizeof(int), hipHostMallocDefault));
   HIP_TRY(hipHostMalloc((void**)&stage_order, (size_t)NW * sizeof(int), hipHostMallocDefault));
@@ -394,6 +397,7 @@ int b2g_batch::alloc() {
     int dev = 0, cus = 0;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    flow_max_blocks = flow_resident_blocks(cus);
     std::vector<uint32_t> all_cus((size_t)std::max(1, (cus + 31) / 32), 0xffffffffu);
     if (hipExtStreamCreateWithCUMask(&side, (uint32_t)all_cus.size(), all_cus.data()) != hipSuccess) {
       // no queue of its own to be had (many live batches): a shared one
@@ -1055,10 +1059,12 @@ void b2g_batch::enqueue_colour_groups() {
 // The coming step's sweeps may be ordered by data: the bodies' flow states
 // exist from the first such step on (a batch that only ever takes the
 // per-world solver does without their 256 bytes per body). Without room for
-// them, or past the launches' reach, the step launches its colours one by one.
+// them, past the launches' reach, or soon after one was withdrawn, the step
+// launches its colours one by one.
 void b2g_batch::use_flow() {
   d.flow_on = 0;
   if (sweeps == 1 || !flow_reaches(cap.bodies)) return;
+  if (sweeps == 0 && !flow_rest.take(pinned[kCntWithdrawn])) return;
   const size_t bytes = (size_t)kFlowStride * std::max(cap.bodies, 1);
   for (unsigned long long** p : {&d.fvel, &d.fpos})
     if (!*p && hipMalloc((void**)p, bytes) != hipSuccess) {
@@ -1170,12 +1176,8 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
   // ordered by data instead (b2g_flow.h): an eager step without a serial
   // group, of no more constraints than the launch keeps resident
   const int flow_cons = nnorm ? begins.empty() ? 0 : begins[nnorm - 1] + sizes[nnorm - 1] : 0;
-  // constraints to a wave: few where the waves are few (kFlowSpread waves, one
-  // or two per SIMD), up to one per lane
-  const int per = std::min(kWave, std::max(1, (flow_cons + d.nj + kFlowSpread - 1) / kFlowSpread));
-  const int jblocks = (d.nj + per * kFlowWaves - 1) / (per * kFlowWaves);
-  const int flow_blocks = jblocks + (flow_cons + per * kFlowWaves - 1) / (per * kFlowWaves);
-  const bool flow = d.flow_on && !tail && !has_serial && flow_blocks <= kFlowMaxBlocks && pi <= kFlowMaxPosIters &&
+  const FlowPlan plan = flow_plan(flow_cons, d.nj);
+  const bool flow = d.flow_on && !tail && !has_serial && plan.blocks <= flow_max_blocks && pi <= kFlowMaxPosIters &&
                     (nnorm == 0 || colours[nnorm - 1] < kBodyTab);
   last_sweeps = flow ? 2 : 1;
   const long long flow_wait = sweeps == 2 ? -1 : kFlowEnterTicks;
@@ -1219,9 +1221,9 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
       const LaunchShape wg = shape_for(d.nb);
       launch(B2G_KERNEL_WARM_START, flow_cons, k_warm_gather, wg.grid, wg.block, 0, d);
     }
-    if (flow_blocks > 0)
-      launch(B2G_KERNEL_CONTACT_VELOCITY, (long long)flow_cons * vi, k_flow_velocity, dim3(flow_blocks),
-             dim3(kFlowThreads), 0, d, flow_cons, jblocks, per, vi, flow_wait);
+    if (plan.blocks > 0)
+      launch(B2G_KERNEL_CONTACT_VELOCITY, (long long)flow_cons * vi, k_flow_velocity, dim3(plan.blocks),
+             dim3(kFlowThreads), 0, d, flow_cons, plan.joint_blocks, plan.per, vi, flow_wait);
   } else if (tail) {  // captured steps: the gather, then the colours past the body table and the serial group
     const LaunchShape wg = shape_for(d.nb);
     launch(B2G_KERNEL_WARM_START, -1, k_warm_gather, wg.grid, wg.block, 0, d);
@@ -1257,9 +1259,9 @@ void b2g_batch::enqueue_solve(int vi, int pi, const std::vector<int>& colours, c
     const LaunchShape si = shape_for(std::max(est_cons + d.nj, d.nb));
     hipLaunchKernelGGL(k_store_and_integrate, si.grid, si.block, 0, stream, d, 1);
   }
-  if (flow && flow_blocks > 0 && pi > 0)
-    launch(B2G_KERNEL_CONTACT_POSITION, (long long)flow_cons * pi, k_flow_position, dim3(flow_blocks),
-           dim3(kFlowThreads), 0, d, flow_cons, jblocks, per, pi, flow_wait);
+  if (flow && plan.blocks > 0 && pi > 0)
+    launch(B2G_KERNEL_CONTACT_POSITION, (long long)flow_cons * pi, k_flow_position, dim3(plan.blocks),
+           dim3(kFlowThreads), 0, d, flow_cons, plan.joint_blocks, plan.per, pi, flow_wait);
   for (int it = 0; it < pi && !flow; ++it) {  // each launch applies the island early exit itself
     contact_sweep(B2G_KERNEL_CONTACT_POSITION, k_contact_position, k_sweep_tail<kTailPosition>, it);
     joint_sweep(k_joint_position, it);

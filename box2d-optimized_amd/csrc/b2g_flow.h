@@ -22,23 +22,20 @@
 // placed within `wait` clock ticks (the GPU is busy with other work), one
 // workgroup withdraws the launch: the others leave, and it sweeps the colours
 // by itself, with barriers. Go and withdrawal are one compare-and-swap, so
-// exactly one happens, before any constraint is touched.
+// exactly one happens, before any constraint is touched. Withdrawals are
+// counted, and the host lets steps rest from these launches after one
+// (FlowRest).
 #pragma once
 
 #include "b2g_kernels.h"
 
 namespace b2g {
 
-constexpr int kFlowThreads = 256;
-constexpr int kFlowWaves = kFlowThreads / kWave;
-// Workgroups of a flow launch at most: two per CU (128 registers per lane
-// allow four), so that two batches on two streams still fit together.
-constexpr int kFlowMaxBlocks = 512;
+static_assert(kFlowLanes == kWave);
 // words of Dev::flow_ctl: the velocity launch's (arrivals, go), the position
 // launch's, then the position launch's barrier counts, one per iteration
 constexpr int kFlowVel = 0, kFlowPos = 2, kFlowBar = 4;
 constexpr int kFlowMaxPosIters = kFlowCtl - kFlowBar;
-constexpr int kFlowSpread = 1024;
 enum FlowGo : int { kFlowWait = 0, kFlowRun = 1, kFlowWithdrawn = 2 };
 constexpr long long kFlowEnterTicks = 100000;       // 1 ms of the 100 MHz clock
 // Polls of a wait in which nothing comes, one memory round trip (0.5 us) each,
@@ -374,7 +371,10 @@ __global__ void __launch_bounds__(kFlowThreads, 4) k_flow_velocity(Dev d, int co
   if (threadIdx.x == 0) flow_count_in(ctl, (int)gridDim.x + (wait < 0 ? 1 : 0));  // (wait < 0: never complete)
   bool sole;
   if (!flow_enter(ctl, wait, &sole)) {
-    if (sole) flow_velocity_alone(d, vi);
+    if (sole) {
+      if (threadIdx.x == 0) ++d.cnt[kCntWithdrawn];
+      flow_velocity_alone(d, vi);
+    }
     return;
   }
   const bool joints = (int)blockIdx.x < jblocks;
@@ -588,7 +588,10 @@ __global__ void __launch_bounds__(kFlowThreads, 4) k_flow_position(Dev d, int co
   if (threadIdx.x == 0) flow_count_in(ctl, (int)gridDim.x + (wait < 0 ? 1 : 0));
   bool sole;
   if (!flow_enter(ctl, wait, &sole)) {
-    if (sole) flow_position_alone(d, pi);
+    if (sole) {
+      if (threadIdx.x == 0) ++d.cnt[kCntWithdrawn];
+      flow_position_alone(d, pi);
+    }
     return;
   }
   int* bar = d.flow_ctl + kFlowBar;

@@ -75,6 +75,8 @@ constexpr int kFlowCtl = 64;
 constexpr int kGroupThreads = 1024, kGroupSlots = 2048, kGroupBodies = 4096;
 constexpr int kWorldClasses = 13;
 constexpr int kCntClass = 16;  // cnt[16 + class]: worlds in each class's list
+constexpr int kCntWithdrawn = kCntClass + kWorldClasses;  // flow launches withdrawn so far
+static_assert(kCntWithdrawn < kCntColOff, "the colour offsets follow");
 constexpr int kPairClass = kWorldClasses - 2;  // one world, two or more contacts to a lane
 __device__ __host__ __forceinline__ constexpr int class_worlds(int c) {  // 16, 12, 10, 8, 7 .. 1, 1
   return c == 0 ? 16 : c == 1 ? 12 : c == 2 ? 10 : c == kPairClass ? 1 : 11 - c;

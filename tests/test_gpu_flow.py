@@ -131,6 +131,22 @@ def test_gpu_a_jointed_body_that_turns_dynamic_gets_a_place_in_its_joints_order(
     assert np.array_equal(ref.joints(sc.joint_count).view(np.uint8), b.joints(sc.joint_count).view(np.uint8))
 
 
+def test_gpu_steps_after_a_withdrawn_launch_take_a_launch_per_colour(engine):
+    """A launch without room for its workgroups costs a millisecond and one workgroup's sweeps: the steps after
+    it do without, and try again later. The states are a launch per colour's all the way."""
+    scenes = [S.gas_and_chains(300, 6, 12, seed=7, half=40.0)]
+    ref, b = engine.Batch.from_scenes(scenes), engine.Batch.from_scenes(scenes)
+    ref.set_option(engine.OPT_SWEEPS, 1)
+    took = []
+    for k in range(300):
+        b.set_option(engine.OPT_SWEEPS, 2 if k == 5 else 0)  # (2: the workgroups give up their places)
+        ref.advance(1)
+        b.advance(1)
+        took.append(b.get_option(engine.OPT_LAST_SWEEPS))
+    assert took == [2] * 6 + [1] * 256 + [2] * 38
+    assert np.array_equal(ref.bodies().view(np.uint8), b.bodies().view(np.uint8))
+
+
 def test_gpu_a_phase_of_many_seconds_is_no_stall(engine):
     """Twenty spokes on one hub, their sweeps a chain of twenty updates an iteration, for so many iterations that
     the launch takes seconds and the bodies' update counts wrap their 16 bits many times."""
