@@ -1057,13 +1057,15 @@ void b2g_batch::enqueue_colour_groups() {
 }
 
 // The coming step's sweeps may be ordered by data: the bodies' flow states
-// exist from the first such step on (a batch that only ever takes the
-// per-world solver does without their 256 bytes per body). Without room for
-// them, past the launches' reach, or soon after one was withdrawn, the step
-// launches its colours one by one.
+// exist from the first such step on (a batch whose worlds are solved in
+// workgroups does without their 256 bytes per body). Without room for them,
+// past the launches' reach, with more constraints in the last step than they
+// keep resident, or soon after one was withdrawn, the step launches its
+// colours one by one.
 void b2g_batch::use_flow() {
   d.flow_on = 0;
   if (sweeps == 1 || !flow_reaches(cap.bodies)) return;
+  if (flow_plan(est_cons, d.nj).blocks > flow_max_blocks) return;
   if (sweeps == 0 && !flow_rest.take(pinned[kCntWithdrawn])) return;
   const size_t bytes = (size_t)kFlowStride * std::max(cap.bodies, 1);
   for (unsigned long long** p : {&d.fvel, &d.fpos})
@@ -1659,7 +1661,7 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
   const bool one = one_world_launch();
   const bool classes = use_classes() || one;
   d.classes_on = classes ? 1 : 0;
-  if (!use_per_world()) use_flow();
+  if (!use_per_world() && !one) use_flow();  // (a single world that outgrows the classes: a launch per colour)
   enqueue_collide_and_colour_eager();
   d.classes_on = 0;
   if (prof_on) HIP_TRY(hipEventRecord(ev[1], stream));

@@ -168,3 +168,15 @@ def test_gpu_a_phase_of_many_seconds_is_no_stall(engine):
         batches.append(b)
     assert np.array_equal(batches[0].bodies().view(np.uint8), batches[1].bodies().view(np.uint8))
     assert np.isfinite(batches[0].bodies()["v"]).all()
+
+
+def test_gpu_a_world_solved_in_a_workgroup_keeps_no_flow_states(engine):
+    """A single world that fits a workgroup does without the bodies' flow states (256 bytes each, and their
+    stores in every step): the step in which it outgrows the workgroup takes a launch per colour."""
+    b = engine.Batch.from_scenes([S.random_pile(1700, seed=7, half_w=24.0, height=130.0)])
+    paths = []
+    while len(paths) < 400 and paths[-2:] != [(1, 2)] * 2:
+        b.advance(1)
+        paths.append((b.get_option(engine.OPT_LAST_SOLVER), b.get_option(engine.OPT_LAST_SWEEPS)))
+    out = [k for k, p in enumerate(paths) if p[0] == 1]
+    assert paths[0][0] == 2 and out and paths[out[0]] == (1, 1) and paths[-1] == (1, 2)
