@@ -229,6 +229,7 @@ struct b2g_batch {
   int world_block = 0;       // B2G_OPT_WORLD_BLOCK (0: the classes of b2g_worlds.h)
   int world_lds = -1;        // B2G_OPT_WORLD_LDS
   int class_count[kWorldClasses] = {};  // worlds per class, as the step read them
+  int large_worlds = 0;      // worlds past every class but the last in the last step by classes
   int last_path = 0;         // 1 colour-major sweeps, 2 per-world, 3 cells
 
   int alloc();
@@ -1415,11 +1416,16 @@ bool b2g_batch::one_world_launch() const {
          est_cons <= class_slots(kOneWorldClass);
 }
 
-// Every active world's solve: one launch for the classes and, beside it on
-// the side stream, the largest worlds. Sized by the class counts the step has
-// read, so captured steps keep k_solve_worlds (a graph also replays its
-// branches one after the other: 1000 worlds, a replayed step 1.2 ms against
-// 1.1).
+// Every active world's solve, sized by the class counts the step has read (so
+// captured steps keep k_solve_worlds; a graph also replays its branches one
+// after the other: 1000 worlds, a replayed step 1.2 ms against 1.1). The
+// worlds past the classes are the longest: their set-up and solve go on the
+// main stream, without waiting for another queue. The classes' launch runs
+// beside the solve on the side stream, and is submitted after the set-up: its
+// workgroups take a whole CU each for 100 us and more, and the set-up's three
+// short launches had to wait for them one after the other (1000 settled worlds
+// of 290 contacts on average, 5 of them past the classes: a step of 0.90 ms
+// when both were submitted at once, 0.81 so; 50 worlds of 560: 0.51 and 0.49).
 void b2g_batch::launch_classes(int vi, int pi) {
   tbegin(B2G_KERNEL_SOLVER);
   const int rounds = rounds_pending;
@@ -1433,31 +1439,33 @@ void b2g_batch::launch_classes(int vi, int pi) {
   int blocks = 0;
   for (int c = 0; c < kPairClass; ++c) blocks += class_blocks(class_count[c], c, threads == kGroupThreads);
   const int pairs = class_count[kPairClass], over = class_count[last];
-  // the largest worlds first, on the side stream beside the others
   const bool fork = over + pairs > 0 && blocks > 0;
-  hipStream_t st = fork ? side : stream;
+  const int* list = d.wclass + (size_t)last * d.nw;
+  if (over > 0) {
+    hipLaunchKernelGGL(k_world_colour_sort, dim3(over), dim3(kBlock), 0, stream, d, 0, list);
+    hipLaunchKernelGGL(k_world_islands<kIslandLdsMid>, dim3(over), dim3(512), 0, stream, d, list);
+    hipLaunchKernelGGL(k_worlds_init, dim3(over, 16), dim3(kBlock), 0, stream, d, list);
+  }
   if (fork) {
     (void)hipEventRecord(fork_ev, stream);
     (void)hipStreamWaitEvent(side, fork_ev, 0);
   }
   if (over > 0) {
-    const int* list = d.wclass + (size_t)last * d.nw;
-    hipLaunchKernelGGL(k_world_colour_sort, dim3(over), dim3(kBlock), 0, st, d, 0, list);
-    hipLaunchKernelGGL(k_world_islands<kIslandLdsMid>, dim3(over), dim3(512), 0, st, d, list);
-    hipLaunchKernelGGL(k_worlds_init, dim3(over, 16), dim3(kBlock), 0, st, d, list);
     const int bodies = std::min(max_world_bodies, kLdsBodyLimit);
-    hipLaunchKernelGGL(k_solve_worlds<true>, dim3(over), dim3(1024), sizeof(float4) * (size_t)bodies, st, d, vi, pi,
-                       0, list, bodies);
+    hipLaunchKernelGGL(k_solve_worlds<true>, dim3(over), dim3(1024), sizeof(float4) * (size_t)bodies, stream, d, vi,
+                       pi, 0, list, bodies);
   }
   if (pairs > 0)
-    hipLaunchKernelGGL((k_step_worlds<kPairThreads, kGroupSlots / kPairThreads>), dim3(pairs), dim3(kPairThreads), 0, st,
-                       d, vi, pi, blocks > 0 ? 0 : rounds, kPairClass, kPairClass);
-  if (fork) (void)hipEventRecord(join_ev, side);
+    hipLaunchKernelGGL((k_step_worlds<kPairThreads, kGroupSlots / kPairThreads>), dim3(pairs), dim3(kPairThreads), 0,
+                       stream, d, vi, pi, blocks > 0 ? 0 : rounds, kPairClass, kPairClass);
   // (with no world in any class the launch still moves the claim-round base on)
   if (blocks > 0 || pairs <= 0)
-    hipLaunchKernelGGL((k_step_worlds<kGroupThreads, 1>), dim3(std::max(blocks, 1)), dim3(threads), 0, stream, d, vi,
-                       pi, rounds, 0, kPairClass - 1);
-  if (fork) (void)hipStreamWaitEvent(stream, join_ev, 0);
+    hipLaunchKernelGGL((k_step_worlds<kGroupThreads, 1>), dim3(std::max(blocks, 1)), dim3(threads), 0,
+                       fork ? side : stream, d, vi, pi, rounds, 0, kPairClass - 1);
+  if (fork) {
+    (void)hipEventRecord(join_ev, side);
+    (void)hipStreamWaitEvent(stream, join_ev, 0);
+  }
   tend(B2G_KERNEL_SOLVER, est_cons);
 }
 
@@ -1660,7 +1668,12 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
   d.segs = pairs_current && worlds_contiguous ? 1 : 0;
   const bool one = one_world_launch();
   const bool classes = use_classes() || one;
-  d.classes_on = classes ? 1 : 0;
+  // (a world past the classes takes k_solve_worlds for longer than a smaller
+  // world does: beside one, as in the last step, the last but one class joins
+  // its launch instead of queueing one of its own. Settled: 50 worlds of up to
+  // 2900 contacts 0.72 ms a step with both launches, 0.51 so; without a world
+  // past the classes 0.37 with the class's own launch, 0.46 in k_solve_worlds)
+  d.classes_on = !classes ? 0 : !one && large_worlds > 0 ? 2 : 1;
   if (!use_per_world() && !one) use_flow();  // (a single world that outgrows the classes: a launch per colour)
   enqueue_collide_and_colour_eager();
   d.classes_on = 0;
@@ -1671,6 +1684,7 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
     if ((rc = read_counters())) return rc;
     if ((rc = status_error())) return rc;  // an earlier (asynchronous) step overflowed
     for (int c = 0; c < kWorldClasses; ++c) class_count[c] = pinned[kCntClass + c];
+    large_worlds = pinned[kCntLarge];
     est_cons = pinned[C_CONS];
     // (the world outgrew the classes: the colour sweeps below)
     if (one) per_world = est_cons <= class_slots(kOneWorldClass) && class_count[kWorldClasses - 1] == 0;

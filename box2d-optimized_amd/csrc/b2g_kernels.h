@@ -76,7 +76,8 @@ constexpr int kGroupThreads = 1024, kGroupSlots = 2048, kGroupBodies = 4096;
 constexpr int kWorldClasses = 13;
 constexpr int kCntClass = 16;  // cnt[16 + class]: worlds in each class's list
 constexpr int kCntWithdrawn = kCntClass + kWorldClasses;  // flow launches withdrawn so far
-static_assert(kCntWithdrawn < kCntColOff, "the colour offsets follow");
+constexpr int kCntLarge = kCntWithdrawn + 1;  // active worlds past the last but one class
+static_assert(kCntLarge < kCntColOff, "the colour offsets follow");
 constexpr int kPairClass = kWorldClasses - 2;  // one world, two or more contacts to a lane
 __device__ __host__ __forceinline__ constexpr int class_worlds(int c) {  // 16, 12, 10, 8, 7 .. 1, 1
   return c == 0 ? 16 : c == 1 ? 12 : c == 2 ? 10 : c == kPairClass ? 1 : 11 - c;
@@ -106,7 +107,7 @@ struct Dev {
   int2* wbody;    // body range of each world (worlds laid out world after world)
   int* worder;    // worlds by decreasing size: the per-world solver's block order
   int* wact;      // the worlds active in the step, in the same order (mostly idle batches)
-  int classes_on; // this step lists the active worlds by class (b2g_worlds.h)
+  int classes_on; // this step lists the active worlds by class (b2g_worlds.h); 2: the last but one class with the last
   int* wclass;    // kWorldClasses lists of nw: the active worlds of each class
   int* wcol;      // per world: kColourSlots + 1 slot offsets of its colour groups
   int* wcolmax;   // per world: highest normal colour used this step (-1: none)
@@ -345,6 +346,7 @@ __device__ __forceinline__ void reset_colour_counters(const Dev& d) {
   for (int c = threadIdx.x; c < kColourSlots; c += blockDim.x) d.col_count[c] = 0;
   if (threadIdx.x < kFlowCtl) d.flow_ctl[threadIdx.x] = 0;
   if (threadIdx.x < kWorldClasses) d.cnt[kCntClass + threadIdx.x] = 0;
+  if (threadIdx.x == 0) d.cnt[kCntLarge] = 0;
   if (threadIdx.x == 0) {
     d.cnt[C_REMAIN] = 0;
     d.cnt[C_PENDING] = 0;
@@ -605,6 +607,8 @@ __global__ void __launch_bounds__(kBlock) k_colour_init(Dev d, int K) {
       const int nb = d.wbody[w].y - d.wbody[w].x;
       int c = 0;
       while (c < kWorldClasses - 1 && (t.y - t.x > class_slots(c) || nb > class_bodies(c))) ++c;
+      if (c == kWorldClasses - 1) atomicAdd(&d.cnt[kCntLarge], 1);
+      if (c == kPairClass && d.classes_on == 2) c = kWorldClasses - 1;
       d.wclass[(size_t)c * d.nw + atomicAdd(&d.cnt[kCntClass + c], 1)] = w;
     }
   }

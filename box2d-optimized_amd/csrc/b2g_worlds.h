@@ -23,9 +23,11 @@
 // each, and steps the colours of all its worlds at once. (A launch per class
 // left the small classes waiting for each other, 60 us each whatever their
 // size.) Worlds of 1025 to 2048 contacts take a workgroup of 512 lanes with
-// four constraints to a lane, which spills and costs 122 us for the largest of
-// 64 worlds against k_solve_worlds' 159; all worlds that way cost the smaller
-// ones 25%. Worlds past 2048 contacts or 4096 bodies take k_solve_worlds.
+// four constraints to a lane, which spills: 122 us for the largest of 64 worlds
+// that still fall, 230 us settled, against 159 and about 270 for the set-up
+// launches and k_solve_worlds; all worlds that way cost the smaller ones 25%.
+// Worlds past 2048 contacts or 4096 bodies take k_solve_worlds, and those of
+// 1025 to 2048 with them where the last step had any (Dev::classes_on).
 #pragma once
 
 #include "b2g_kernels.h"

@@ -107,3 +107,22 @@ def test_gpu_worlds_past_the_largest_class_keep_the_claim_rounds(engine):
         assert np.array_equal(a.contact_colours(n), b.contact_colours(n)), k
     _same(a, b, "end")
     assert a.counts().touching > 2048  # (the large world is past the largest class by far)
+
+
+def test_gpu_worlds_of_the_last_classes_share_a_launch_while_both_are_active(engine):
+    """A world of 1025 to 2048 contacts is solved in its own class's launch, or with the worlds past it where the
+    step before had one: both come and go here."""
+    scenes = [S.pyramid(30), S.pyramid(44), S.pyramid(34)] + [S.batch_world(i, 40 + 50 * i) for i in range(6)]
+    a, b = _pair(engine, scenes)
+    a.advance(3)
+    b.advance(3)
+    dt = np.float32(1.0 / 60.0)
+    for k, off in enumerate([(), (1,), (1,), (0, 2), (), (0, 1, 2), (), (3, 4, 5, 6, 7, 8), (), (1,), ()]):
+        for x in (a, b):
+            x.set_world_params(0, [engine.WorldParams(g, dt, 1.0, 1, int(w not in off))
+                                   for w, g in enumerate(x.gravity)])
+            x.step(8, 3, 0)
+        assert a.get_option(engine.OPT_LAST_SOLVER) == 2
+        _same(a, b, (k, off))
+    n = len(a.contacts())
+    assert np.array_equal(a.contact_colours(n), b.contact_colours(n))
