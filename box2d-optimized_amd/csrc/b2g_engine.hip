@@ -24,6 +24,7 @@
 #include "b2g_flow.h"
 #include "b2g_worlds.h"
 #include "b2g_joints.h"
+#include "b2g_world_rule.h"
 
 using namespace b2g;
 
@@ -212,6 +213,7 @@ struct b2g_batch {
   bool keep_idle = true;     // B2G_OPT_KEEP_IDLE
   int pair_search = 0;       // B2G_OPT_PAIR_SEARCH
   int sweeps = 0;            // B2G_OPT_SWEEPS
+  int cus = 0;               // compute units of the device
   int flow_max_blocks = 0;   // workgroups of a flow launch that the device keeps resident
   FlowRest flow_rest;
   int last_sweeps = 0;       // 1 a launch per colour, 2 ordered by data (k_flow_velocity, k_flow_position)
@@ -395,7 +397,7 @@ int b2g_batch::alloc() {
     // process gets a few hardware queues that its streams share, and two
     // streams on one queue run one after the other; a stream created with a
     // CU mask gets a queue of its own, and this mask names every CU.
-    int dev = 0, cus = 0;
+    int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     flow_max_blocks = flow_resident_blocks(cus);
@@ -1389,15 +1391,13 @@ bool b2g_batch::use_per_world() const {
 // 8192 bodies at most, fits)
 constexpr int kLdsBodyLimit = (156 * 1024) / 16;
 constexpr int kSmallWorldLds = 512;
-constexpr int kWorldBlockDefault = 256;
 
-int b2g_batch::world_block_now() const { return world_block > 0 ? world_block : kWorldBlockDefault; }
+int b2g_batch::world_block_now() const { return world_block > 0 ? world_block : captured_world_lanes(d.nw, cus); }
 
-// (workgroups of 64 to 512 with and without the bodies in LDS, captured steps
-// of settled worlds: 1000 worlds of a few to hundreds of bodies take 0.90 ms at
-// 256 with the stage, 1.00 without, 1.02 and 1.03 at 128; 4096 equal ones 3.60
-// and 3.78, 3.54 and 3.94 at 128; 64 large ones 0.43 and 0.45, 0.51 and 0.54. A
-// world past a launch's stage reads its bodies from global memory)
+// (captured steps of settled worlds with and without the bodies in LDS: 1000
+// worlds of a few to hundreds of bodies take 0.90 and 1.00 ms at 256 lanes, 4096
+// equal ones 3.54 and 3.94 at 128, 64 large ones 0.43 and 0.45 at 512. A world
+// past a launch's stage reads its bodies from global memory)
 bool b2g_batch::world_lds_now() const { return world_lds > 0 || (world_lds < 0 && world_block == 0); }
 
 // The per-world solver by classes (b2g_worlds.h), unless the caller picked a

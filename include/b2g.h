@@ -296,9 +296,9 @@ int b2g_time_kernel(b2g_batch* batch, int32_t kernel);
  * b2g_download_contact_colours as phase * 65536 + colour; on request only).
  * B2G_OPT_WORLD_BLOCK: threads per world workgroup, 0 = the engine's choice:
  * eager steps solve worlds in workgroups by their contact counts, captured
- * steps in workgroups of one fixed size. A size given here, or a B2G_OPT_WORLD_LDS
- * of 0 or 1, holds for both. B2G_OPT_TUNED_WORLD_BLOCK is the size of a captured
- * step's workgroups.
+ * steps in workgroups of one size, the wider the fewer worlds there are. A
+ * size given here, or a B2G_OPT_WORLD_LDS of 0 or 1, holds for both.
+ * B2G_OPT_TUNED_WORLD_BLOCK is the size of a captured step's workgroups.
  * Read-only: B2G_OPT_TUNED_WORLD_BLOCK, B2G_OPT_LAST_SOLVER (1 colours,
  * 2 worlds, 3 cells), B2G_OPT_PER_WORLD_ELIGIBLE. No reference counterpart. */
 enum { B2G_SOLVER_AUTO = 0, B2G_SOLVER_COLOURS = 1, B2G_SOLVER_WORLDS = 2, B2G_SOLVER_CELLS = 3 };

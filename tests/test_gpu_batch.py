@@ -339,7 +339,7 @@ def test_gpu_graph_steps_async_batch(engine):
 
 def test_gpu_per_world_solver_matches_colour_sweeps_bitexact(engine):
     """The one-workgroup-per-world solver gives the colour-major sweeps'
-    results bit for bit, for every workgroup size the autotuner may pick."""
+    results bit for bit, for every workgroup size a caller or the engine may pick."""
     scenes = _mixed_scenes()[:2] + [S.batch_world(i, 50 + 30 * i) for i in range(10)]
     scenes = [s for s in scenes if s.joint_count == 0]
     ref = engine.Batch.from_scenes(scenes)
@@ -362,15 +362,15 @@ def test_gpu_per_world_solver_matches_colour_sweeps_bitexact(engine):
 
 
 def test_gpu_per_world_autotune_and_graph(engine):
-    """Auto mode picks the per-world solver for a batch of small worlds, the
-    autotuner settles on a block size within ten steps, and graph replays of
-    the per-world step match eager steps."""
+    """Auto mode picks the per-world solver for a batch of small worlds, its
+    captured steps take the workgroup size that the number of worlds asks for,
+    and graph replays of the per-world step match eager steps."""
     scenes = [S.batch_world(i, 60 + 20 * i) for i in range(16)]
     a = engine.Batch.from_scenes(scenes).advance(12)
     assert a.get_option(engine.OPT_LAST_SOLVER) == 2
     tuned = a.get_option(engine.OPT_TUNED_WORLD_BLOCK)
-    print("autotuned world block:", tuned, flush=True)
-    assert tuned in (64, 128, 256, 512, 1024)
+    print("captured world block:", tuned, flush=True)
+    assert tuned == 1024  # 16 worlds: a compute unit for each
     b = engine.Batch.from_scenes(scenes).advance(12)
     for k in range(20):
         a.step(8, 3, 0)
