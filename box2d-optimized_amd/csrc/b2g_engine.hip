@@ -1668,12 +1668,9 @@ int b2g_batch::eager_step(int vi, int pi, unsigned flags) {
   d.segs = pairs_current && worlds_contiguous ? 1 : 0;
   const bool one = one_world_launch();
   const bool classes = use_classes() || one;
-  // (a world past the classes takes k_solve_worlds for longer than a smaller
-  // world does: beside one, as in the last step, the last but one class joins
-  // its launch instead of queueing one of its own. Settled: 50 worlds of up to
-  // 2900 contacts 0.72 ms a step with both launches, 0.51 so; without a world
-  // past the classes 0.37 with the class's own launch, 0.46 in k_solve_worlds)
-  d.classes_on = !classes ? 0 : !one && large_worlds > 0 ? 2 : 1;
+  const int largest = class_count[kPairClass] + class_count[kWorldClasses - 1];  // the last step's
+  const bool together = !one && pair_class_joins(largest, large_worlds, cus);
+  d.classes_on = !classes ? 0 : together ? 2 : 1;
   if (!use_per_world() && !one) use_flow();  // (a single world that outgrows the classes: a launch per colour)
   enqueue_collide_and_colour_eager();
   d.classes_on = 0;

@@ -22,7 +22,8 @@ struct FlowPlan {
   int per, joint_blocks, blocks;
 };
 inline FlowPlan flow_plan(long long contacts, long long joints) {
-  const int per = (int)std::min<long long>(kFlowLanes, std::max<long long>(1, (contacts + joints + kFlowSpread - 1) / kFlowSpread));
+  const long long even = (contacts + joints + kFlowSpread - 1) / kFlowSpread;
+  const int per = (int)std::min<long long>(kFlowLanes, std::max<long long>(1, even));
   const long long share = (long long)per * kFlowWaves;
   const int jb = (int)((joints + share - 1) / share);
   return FlowPlan{per, jb, jb + (int)((contacts + share - 1) / share)};

@@ -1,5 +1,5 @@
-// b2g_world_rule.h -- the workgroup size of the captured per-world solve. Host
-// code only, without a device header: the CPU tests compile it by itself.
+// b2g_world_rule.h -- rules of the per-world solves' launches. Host code only,
+// without a device header: the CPU tests compile it by itself.
 #pragma once
 
 namespace b2g {
@@ -21,7 +21,28 @@ namespace b2g {
 //   2500 worlds  1.98 / 1.65 / 1.55 / 1.92 / 2.57  (falling 1.33 / 1.17 / 1.21 / 1.64 / 2.31)
 //   4096 worlds  2.56 / 2.21 / 2.25 / 2.96 / 4.09  (falling 1.72 / 1.62 / 1.86 / 2.57 / 3.68)
 constexpr int captured_world_lanes(int worlds, int compute_units) {
-  return worlds <= compute_units ? 1024 : 2 * worlds <= 5 * compute_units ? 512 : worlds <= 10 * compute_units ? 256 : 128;
+  return worlds <= compute_units            ? 1024
+         : 2LL * worlds <= 5LL * compute_units ? 512
+         : worlds <= 10LL * compute_units      ? 256
+                                               : 128;
+}
+
+// Whether the worlds of the last but one class (1025 to 2048 contacts) join
+// the launch of the worlds past the classes in an eager step, going by the
+// last step's counts: `worlds` of both, `past` of them past the classes. A
+// world past them takes k_solve_worlds for longer than a smaller one does, so
+// beside one, and with a CU for each, the class costs nothing there, where its
+// own launch (k_step_worlds, 512 lanes) would queue behind it. With more
+// worlds than CUs the launch is bound by their sum, and the class's own is the
+// faster per world; so it is where no world is past the classes. ms a settled
+// step with a launch of its own / joined:
+//     50 worlds of up to  2900 contacts          0.72 / 0.49
+//     50 worlds of up to  1400 contacts          0.37 / 0.46
+//   1000 worlds, 150 in the two classes          1.49 / 1.21 (both with the classes' launch submitted late)
+//   2500 worlds, 360 in them                     2.14 / 2.23
+//   4096 worlds, 590 in them                     3.09 / 3.39
+constexpr bool pair_class_joins(int worlds, int past, int compute_units) {
+  return past > 0 && worlds <= compute_units;
 }
 
 }  // namespace b2g
