@@ -3272,9 +3272,12 @@ __global__ void __launch_bounds__(kQueryBlock) k_query_aabbs(Dev d, int n, const
 // A ray is a serial walk bound by the latency of its node and shape loads,
 // and the rays of one wavefront diverge at every node: it waits for each of
 // its rays' paths in turn. So only `lanes` lanes of a wavefront hold a ray,
-// few while the rays do not fill the device with wavefronts. Rays through 20k
-// bodies, traversal with its copies, at 4 / 16 / 64 lanes: 64 rays 0.39 / 0.70
-// / 1.05 ms, 4096 rays 0.68 / 0.89 / 1.23 ms, 32768 rays 1.71 / 1.07 / 1.41 ms.
+// few while the rays do not fill the device with wavefronts: n / kRayWaves, at
+// least one. Rays through 20k bodies, a counting walk with its copies, at 1 / 2 /
+// 4 / 8 / 16 / 64 lanes: 64 rays 267 / 338 / 396 / 506 / 691 / 1021 us (takes 1),
+// 4096 rays 494 / 446 / 602 / 723 / 909 / 1240 (takes 2), 8192 rays 737 / 711 /
+// 627 / 880 / 994 / 1261 (takes 4), 32768 rays 2178 / 1828 / 1546 / 1377 / 1047 /
+// 1395 (takes 16).
 __global__ void __launch_bounds__(kWave) k_raycast(Dev d, int n, const float4* __restrict__ segs,
                                                    const int* __restrict__ worlds, int cap, int lanes,
                                                    const int* __restrict__ offs, float4* __restrict__ out,

@@ -400,8 +400,9 @@ int b2g_raycast(b2g_batch* batch, int32_t n, const int32_t* worlds, const float*
 /* The same queries with all their results, one query after the other: the
  * first call runs them (`capacity`: the results of one query that its first
  * pass has room for; any number is found) and gives each query's count and
- * the total, b2g_query_results then writes that many records (int32_t shapes
- * or b2g_ray_hit) to `out`, once, before the batch's next query. */
+ * the total (at most 2^31 - 1, else B2G_ERR_CAPACITY), b2g_query_results then
+ * writes that many records (int32_t shapes or b2g_ray_hit) to `out`, once,
+ * before the batch's next query. */
 int b2g_query_aabbs_list(b2g_batch* batch, int32_t n, const int32_t* worlds, const float* aabbs, int32_t capacity,
                          int32_t* out_counts, int64_t* total);
 int b2g_raycast_list(b2g_batch* batch, int32_t n, const int32_t* worlds, const float* segments, int32_t capacity,
