@@ -22,10 +22,12 @@ Further sections of the same JSON line:
   under a 64 GB memory budget; p50/p99 latency beside throughput.
 
 roofline: HIP events around each run of consecutive launches of the
-dominant kernel (one sweep's per-colour launches), over a further measured
-segment, give its average launch duration. Algorithmic bytes
-per launch are the per-item payloads of the reference's data layout (counted
-once per pass) times the items the launch processed.
+dominant kernel (one launch for all velocity iterations, or one sweep's
+per-colour launches), over a further measured segment, give its average launch
+duration. Algorithmic bytes per launch are the per-item payloads of the
+reference's data layout (counted once per pass that reads them) times the items
+the launch processed. `device_kernel` names the kernel that ran; its measured
+traffic is given where profiles/ holds that kernel's counters.
 
 cpu_baseline: the reference library itself (oracle/_ref, compiled from the
 reference sources) steps the same scene over the same steps on one host core.
@@ -53,11 +55,14 @@ HBM_PEAK_GBS = 8000.0
 #   contact velocity sweep (per solved contact): VC R + impulses W + 2 bodies' velocity R+W
 #   contact position sweep (per solved contact): PC R + 2 bodies' position R+W
 #   pair write (per shape): AABB R + key/index W (+ 8 B per reported pair)
-def item_bytes(kernel: str, geo_bytes: float) -> float:
+# An item of a sweep is one contact in one iteration. A launch per colour reads
+# the constraint in each; a launch of `held` iterations ordered by data reads it
+# (and writes its impulses) once for all of them.
+def item_bytes(kernel: str, geo_bytes: float, held: int = 1) -> float:
     return {
         "narrowphase": 2 * 16 + 2 * geo_bytes + 64 + 64,
-        "contact_velocity": 168 + 16 + 2 * 2 * 12,
-        "contact_position": 88 + 2 * 2 * 12,
+        "contact_velocity": (168 + 16) / held + 2 * 2 * 12,
+        "contact_position": 88 / held + 2 * 2 * 12,
         "pairs_write": 16 + 8,
     }[kernel]
 
@@ -81,16 +86,15 @@ def step_bytes(B: float, S: float, C: float, T: float, P: float, J: float, geo: 
 
 
 def measured_traffic_ratio(kernel: str, workload: str):
-    """HBM bytes / algorithmic bytes per launch of `kernel`, from the committed
-    rocprofv3 --pmc summary (FETCH_SIZE and WRITE_SIZE runs scaled by a plain
-    copy kernel), or None when that kernel/workload was not measured."""
+    """HBM bytes / algorithmic bytes per launch of the device kernel `kernel`,
+    from the committed rocprofv3 --pmc summary (FETCH_SIZE and WRITE_SIZE runs
+    scaled by a plain copy kernel), or None when that kernel/workload was not
+    measured."""
     path = os.path.join(REPO, "profiles", f"pmc_traffic_{workload}.md")
-    if kernel != "contact_velocity" or not os.path.exists(path):
+    if not os.path.exists(path):
         return None
-    for line in open(path):
-        if line.startswith("traffic_ratio:"):
-            return float(line.split(":")[1])
-    return None
+    found = dict(line.strip().split(": ", 1) for line in open(path) if line.startswith(("kernel: ", "traffic_ratio: ")))
+    return float(found["traffic_ratio"]) if found.get("kernel") == kernel else None
 
 
 def workloads(pkg):
@@ -432,7 +436,13 @@ def main():
     k_ms, k_launches, k_items = batch.kernel_time()
     batch.time_kernel(-1)
     geo = mean_geometry_bytes(scene)
-    per_item = item_bytes(args.kernel, geo)
+    # the sweeps as the timed steps ran them (always eager): a launch per colour, or one for all iterations
+    ordered = batch.get_option(eng.OPT_LAST_SOLVER) == 1 and batch.get_option(eng.OPT_LAST_SWEEPS) == 2
+    held = {"contact_velocity": 8, "contact_position": 3}.get(args.kernel, 1) if ordered else 1
+    device_kernel = {"contact_velocity": "k_flow_velocity" if ordered else "k_contact_velocity",
+                     "contact_position": "k_flow_position" if ordered else "k_contact_position",
+                     "narrowphase": "k_narrowphase", "pairs_write": "pair search"}[args.kernel]
+    per_item = item_bytes(args.kernel, geo, held)
     avg_ms = k_ms / max(k_launches, 1)
     bytes_per_launch = per_item * k_items / max(k_launches, 1)
     achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
@@ -460,7 +470,7 @@ def main():
         serving = serving_section(pkg, args.serve_worlds, args.serve_rate, args.serve_seconds,
                                   args.serve_budget_gb, not args.eager)
 
-    ratio = measured_traffic_ratio(args.kernel, args.workload)
+    ratio = measured_traffic_ratio(device_kernel, args.workload)
     value = ndyn * args.steps / elapsed
     line = {
         "metric": "body-steps/s on 1 GPU vs host CPU (20k pile)",
@@ -483,7 +493,7 @@ def main():
                    "launch": "eager" if args.eager else "hipGraph replay of the whole step",
                    "graph_steps": counts.graph_steps, "serial_constraints": counts.serial,
                    "solver": solver_path},
-        "roofline": {"bound": "hbm", "kernel": args.kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
+        "roofline": {"bound": "hbm", "kernel": args.kernel, "device_kernel": device_kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": (ratio * bytes_per_launch) if ratio else None,
                      "traffic_source": (f"profiles/pmc_traffic_{args.workload}.md: measured HBM/algorithmic "
