@@ -1408,18 +1408,23 @@ bool b2g_batch::use_classes() const {
 
 // One joint-free world whose solve fits a workgroup of b2g_worlds.h, going by
 // the last step's constraints (the step checks its own): a 20-row pyramid's
-// step with its read-back takes 186 us, with the flow launches 269. Past the
-// largest class the flow launches spread over the device.
+// step with its read-back takes 205 us, with the flow launches 269. Past the
+// largest class the flow launches spread over the device. While a caller times
+// the sweeps (b2g_time_kernel) the world takes them: the workgroup's launch
+// has none to time.
 bool b2g_batch::one_world_launch() const {
+  const bool sweeps_timed = timed_kernel == B2G_KERNEL_WARM_START || timed_kernel == B2G_KERNEL_CONTACT_VELOCITY ||
+                            timed_kernel == B2G_KERNEL_CONTACT_POSITION;
   return solver_mode == B2G_SOLVER_AUTO && d.nw == 1 && per_world_ok && !d.sleep_on && world_block == 0 &&
-         world_lds < 0 && sweeps == 0 && max_world_bodies <= class_bodies(kOneWorldClass) &&
+         world_lds < 0 && sweeps == 0 && !sweeps_timed && max_world_bodies <= class_bodies(kOneWorldClass) &&
          est_cons <= class_slots(kOneWorldClass);
 }
 
-// Every active world's solve, sized by the class counts the step has read (so
-// captured steps keep k_solve_worlds; a graph also replays its branches one
-// after the other: 1000 worlds, a replayed step 1.2 ms against 1.1). The
-// worlds past the classes are the longest: their set-up and solve go on the
+// Every active world's solve, sized by the class counts the step has read.
+// (Captured steps keep k_solve_worlds: with one launch of these kernels for
+// each class, sized to hold every world, 1000 worlds took 1.2 ms a replayed
+// step against 1.1. A fixed grid that strides over the counts on the device
+// has not been built.) The worlds past the classes are the longest: their set-up and solve go on the
 // main stream, without waiting for another queue. The classes' launch runs
 // beside the solve on the side stream, and is submitted after the set-up: its
 // workgroups take a whole CU each for 100 us and more, and the set-up's three

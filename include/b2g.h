@@ -267,8 +267,11 @@ int b2g_get_counts(b2g_batch* batch, b2g_counts* out);
 /* Timing of every launch of one kernel during the following steps (-1 =
  * off): HIP events around each run of consecutive launches of that kernel
  * (the per-colour launches of one sweep, or a single launch). The contact
- * sweeps are the per-colour launches (not the launch shared by the small
- * trailing colours). b2g_kernel_time returns the summed device time, the
+ * sweeps are the launch for all iterations of a phase where the step orders
+ * them by data (B2G_OPT_LAST_SWEEPS 2), else the per-colour launches (not the
+ * launch shared by the small trailing colours); a single world takes them
+ * while they are timed, also where it is solved in one workgroup otherwise.
+ * Batches solved in workgroups have B2G_KERNEL_SOLVER only. b2g_kernel_time returns the summed device time, the
  * number of launches and the work items they covered (contacts, constraints
  * or shapes). */
 enum {

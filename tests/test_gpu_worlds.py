@@ -126,3 +126,22 @@ def test_gpu_worlds_of_the_last_classes_share_a_launch_while_both_are_active(eng
         _same(a, b, (k, off))
     n = len(a.contacts())
     assert np.array_equal(a.contact_colours(n), b.contact_colours(n))
+
+
+def test_gpu_a_single_world_has_sweeps_to_time(engine):
+    """A small world is solved in one launch, which has no sweeps; a caller who times them gets them, with the
+    same states."""
+    a, b = (engine.Batch.from_scenes([S.pyramid(12)]).advance(30) for _ in range(2))
+    assert a.get_option(engine.OPT_LAST_SOLVER) == 2
+    for kernel in (engine.KERNEL_WARM_START, engine.KERNEL_CONTACT_VELOCITY, engine.KERNEL_CONTACT_POSITION,
+                   engine.KERNEL_NARROWPHASE, engine.KERNEL_SOLVER):
+        a.time_kernel(kernel)
+        for x in (a, b):
+            for _ in range(5):
+                x.step(8, 3, 0)
+        ms, launches, items = a.kernel_time()
+        assert launches >= 5 and ms > 0 and items > 0, kernel
+        a.time_kernel(-1)
+        _same(a, b, kernel)
+    a.step(8, 3, 0)
+    assert a.get_option(engine.OPT_LAST_SOLVER) == 2
